@@ -93,9 +93,13 @@ def schwarz_block(la, lb):
     return _nsph(la) * _nsph(lb) * _ncart(la) * _ncart(lb)
 
 
-# highest l of the gradient kernels: compile-time instances up to d, the
-# runtime-l kernel of eri_grad_any.hip for classes with f shells
+# highest l of the gradient kernels
 GRAD_MAX_L = 3
+
+
+def grad_coop(la, lb, lc, ld):
+    """Classes whose gradient runs in the cooperative kernel (csrc/eri_grad_coop.hpp)."""
+    return max(la, lb, lc, ld) > 2
 
 
 def grad_chunks(la, lb, lc, ld):
@@ -159,8 +163,16 @@ def gen_sources():
             if b == k:
                 sw_cases.append(f"  if (c == {b}) {{ {' '.join(sw_calls)} schwarz_fold_cls_{tag}(a, s); return; }}")
                 sb_cases.append(f"  if (c == {b}) return {schwarz_block(la, lb)};")
-            if fcls:  # classes with f shells: the runtime-l gradient kernel
-                gr_cases.append(f"  if (cb == {b} && ck == {k}) {{ launch_grad_any(a, {la}, {lb}, {lc}, {ld}, s); return; }}")
+            # cooperative gradient kernel (a block per quartet)
+            if grad_coop(la, lb, lc, ld):
+                body = ["// generated by build.py", '#include "../../eri_grad_coop.hpp"', "namespace qfe {",
+                        f"void gradc_cls_{tag}(const GradLaunch& a, hipStream_t s) {{ "
+                        f"grad_coop<{la}, {lb}, {lc}, {ld}>(a, s); }}", "}  // namespace qfe"]
+                decls.append(f"void gradc_cls_{tag}(const GradLaunch& a, hipStream_t s);")
+                path = os.path.join(GEN, f"gradc_{tag}.hip")
+                _write_if_changed(path, "\n".join(body) + "\n")
+                files.append(path)
+                gr_cases.append(f"  if (cb == {b} && ck == {k}) {{ gradc_cls_{tag}(a, s); return; }}")
                 continue
             gops = f"GradOps<{la}, {lb}, {lc}, {ld}, true>"
             gnch = grad_chunks(la, lb, lc, ld)
@@ -256,6 +268,8 @@ def _deps(src):
         hs = ["kernels.hpp"]
     elif name.startswith("chunks"):
         hs = core + ["eri_class.hpp"]
+    elif name.startswith("gradc_"):
+        hs = core + ["eri_class.hpp", "eri_coop.hpp", "eri_grad_coop.hpp"]
     elif name.startswith("grad_") or name.startswith("cls_"):
         hs = core + ["eri_class.hpp", "eri_grad.hpp"]
     elif name == "kernels.hip":
@@ -268,8 +282,6 @@ def _deps(src):
         hs = core + ["dfj.hpp"]
     elif name == "eri_dense.hip":
         hs = core + ["dfj.hpp", "eri_dense.hpp"]
-    elif name == "eri_grad_any.hip":
-        hs = core
     else:  # onebody.cpp
         hs = ["host_common.hpp", "sph_coef.inc"]
     out = [os.path.join(CSRC, h) for h in hs]
@@ -339,7 +351,7 @@ def build(jobs=None, force=False, verbose=False):
     os.makedirs(LIB, exist_ok=True)
     ensure_rys_table()
     srcs = [os.path.join(CSRC, f) for f in ("kernels.hip", "engine.cpp", "onebody.cpp", "onebody_gpu.hip", "dfj.hip",
-                                             "eri_dense.hip", "eri_grad_any.hip")] + gen_sources()
+                                             "eri_dense.hip")] + gen_sources()
     objs = []
     with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
         futs = []

@@ -324,7 +324,7 @@ struct Engine {
   DevBuf<double> P_d, J_d, K_d;      // device buffers handed out by qfe_device_buffers (SCF context too)
   DevBuf<double> hP_d, hJ_d, hK_d;   // staging of the host-pointer build (ndm x nbf x nbf)
   DevBuf<double> gP_d;               // gradient densities: [P or P_alpha][P_beta][P_alpha + P_beta]
-  DevBuf<double> sph_d;              // solid-harmonic table kSph (runtime-l gradient kernel)
+  DevBuf<double> sph_d;              // solid-harmonic table kSph (cooperative gradient kernels)
   std::vector<DevBuf<double>> rys_d;
   DevBuf<double> boys_d;
   std::vector<DevBuf<float>> rys32_d;

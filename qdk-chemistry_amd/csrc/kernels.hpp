@@ -96,7 +96,7 @@ struct GradLaunch {
   double kscale;
   double* gJ;             // 3 * natoms, xyz-major
   double* gK;
-  const double* sph;      // device copy of the solid-harmonic table kSph (runtime-l kernel)
+  const double* sph;      // device copy of the solid-harmonic table kSph (cooperative kernels)
 };
 
 struct SchwarzLaunch {
@@ -119,7 +119,4 @@ void launch_schwarz(int pair_cls, bool pure, const SchwarzLaunch& a, hipStream_t
 void launch_grad(int bra_cls, int ket_cls, bool pure, const GradLaunch& a, hipStream_t s);
 // highest shell angular momentum the gradient kernels of this build cover
 int grad_max_l();
-// the gradient of one class pair with runtime angular momenta (classes with
-// f shells; eri_grad_any.hip)
-void launch_grad_any(const GradLaunch& a, int la, int lb, int lc, int ld, hipStream_t s);
 }  // namespace qfe
