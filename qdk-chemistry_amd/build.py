@@ -97,9 +97,18 @@ def schwarz_block(la, lb):
 GRAD_MAX_L = 3
 
 
-def grad_coop(la, lb, lc, ld):
-    """Classes whose gradient runs in the cooperative kernel (csrc/eri_grad_coop.hpp)."""
-    return max(la, lb, lc, ld) > 2
+def grad_coop_tasks(ltot):
+    """Quartets up to which a class without f shells runs in the cooperative
+    gradient kernel (csrc/eri_grad_coop.hpp, a block per quartet) instead of
+    the chunk kernels of csrc/eri_grad.hpp (a thread per quartet and chunk).
+    With few quartets a thread's chain of primitive quartets is the time, and
+    every chunk repeats it: (dp|pp) at 14,376 quartets 4.2 ms in 18 chunks
+    against 0.32 ms.  With many the chunk kernels win, as they read no LDS
+    tables: (dp|pp) at 808,005 quartets 8.1 against 11.1 ms.  The two meet at
+    60-150 thousand quartets up to L = 3 and from L = 6 ((pp|ss) at 135,741:
+    0.56 and 0.54 ms; (dd|dd) at 34,133: 2.3 and 2.6 ms) and near 200-400
+    thousand between ((ds|pp) at 417,355: 3.4 and 3.3 ms)."""
+    return 200000 if 4 <= ltot <= 5 else (100000 if ltot < 4 else 60000)
 
 
 def grad_chunks(la, lb, lc, ld):
@@ -163,16 +172,18 @@ def gen_sources():
             if b == k:
                 sw_cases.append(f"  if (c == {b}) {{ {' '.join(sw_calls)} schwarz_fold_cls_{tag}(a, s); return; }}")
                 sb_cases.append(f"  if (c == {b}) return {schwarz_block(la, lb)};")
-            # cooperative gradient kernel (a block per quartet)
-            if grad_coop(la, lb, lc, ld):
-                body = ["// generated by build.py", '#include "../../eri_grad_coop.hpp"', "namespace qfe {",
-                        f"void gradc_cls_{tag}(const GradLaunch& a, hipStream_t s) {{ "
-                        f"grad_coop<{la}, {lb}, {lc}, {ld}>(a, s); }}", "}  // namespace qfe"]
-                decls.append(f"void gradc_cls_{tag}(const GradLaunch& a, hipStream_t s);")
-                path = os.path.join(GEN, f"gradc_{tag}.hip")
-                _write_if_changed(path, "\n".join(body) + "\n")
-                files.append(path)
-                gr_cases.append(f"  if (cb == {b} && ck == {k}) {{ gradc_cls_{tag}(a, s); return; }}")
+            # cooperative gradient kernel (a block per quartet): every class with
+            # an f shell, the others up to grad_coop_tasks quartets
+            body = ["// generated by build.py", '#include "../../eri_grad_coop.hpp"', "namespace qfe {",
+                    f"void gradc_cls_{tag}(const GradLaunch& a, hipStream_t s) {{ "
+                    f"grad_coop<{la}, {lb}, {lc}, {ld}>(a, s); }}", "}  // namespace qfe"]
+            decls.append(f"void gradc_cls_{tag}(const GradLaunch& a, hipStream_t s);")
+            path = os.path.join(GEN, f"gradc_{tag}.hip")
+            _write_if_changed(path, "\n".join(body) + "\n")
+            files.append(path)
+            few = "" if fcls else f" && a.ntask <= {grad_coop_tasks(ltot)}"
+            gr_cases.append(f"  if (cb == {b} && ck == {k}{few}) {{ gradc_cls_{tag}(a, s); return; }}")
+            if fcls:
                 continue
             gops = f"GradOps<{la}, {lb}, {lc}, {ld}, true>"
             gnch = grad_chunks(la, lb, lc, ld)
@@ -269,7 +280,7 @@ def _deps(src):
     elif name.startswith("chunks"):
         hs = core + ["eri_class.hpp"]
     elif name.startswith("gradc_"):
-        hs = core + ["eri_class.hpp", "eri_coop.hpp", "eri_grad_coop.hpp"]
+        hs = core + ["eri_class.hpp", "eri_grad.hpp", "eri_coop.hpp", "eri_grad_coop.hpp"]
     elif name.startswith("grad_") or name.startswith("cls_"):
         hs = core + ["eri_class.hpp", "eri_grad.hpp"]
     elif name == "kernels.hip":

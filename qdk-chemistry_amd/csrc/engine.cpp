@@ -216,6 +216,11 @@ static unsigned char* noalloc_scratch(int device) {
   return addr.emplace(device, static_cast<unsigned char*>(p)).first->second;
 }
 
+// Copies of the gradient accumulators (6 doubles an atom each) that the
+// gradient kernels' blocks spread their atomics over: with one copy the
+// blocks of a small molecule queue at a few hundred addresses.
+constexpr int kGradCopies = 32;
+
 struct Engine {
   // input
   BasisHost basis;
@@ -288,7 +293,7 @@ struct Engine {
   DevBuf<double> sig_d;     // primitive-quartet screening factor per primitive pair
   DevBuf<float> sig32_d;
   DevBuf<int> sh_atom_d;
-  DevBuf<double> grad_d;    // [2][3 * natoms]
+  DevBuf<double> grad_d;    // [kGradCopies][2][3 * natoms]
   DevBuf<float4> ppos32_d;  // single-precision copies for the FP32 tasks
   DevBuf<float> pk32_d;
   DevBuf<double> Q_d;
@@ -983,7 +988,7 @@ struct Engine {
                           std::to_string(grad_max_l()));
     HIP_CHECK(hipSetDevice(device));
     const size_t nn = (size_t)nbf * nbf;
-    grad_d.alloc(6 * (size_t)natoms);
+    grad_d.alloc(kGradCopies * 6 * (size_t)natoms);
     hipStream_t s = stream;
     // device layout: [P_screen/P_alpha][P_beta][P_total]
     gP_d.alloc(ndm == 1 ? nn : 3 * nn);
@@ -999,7 +1004,7 @@ struct Engine {
       Pj = gP_d.p + 2 * nn;
       Pk2 = gP_d.p + nn;
     }
-    HIP_CHECK(hipMemsetAsync(grad_d.p, 0, sizeof(double) * 6 * natoms, s));
+    HIP_CHECK(hipMemsetAsync(grad_d.p, 0, sizeof(double) * kGradCopies * 6 * natoms, s));
     HIP_CHECK(hipEventRecord(ev[0], s));
     std::vector<long long> bval = screen(gP_d.p, s, false);
     HIP_CHECK(hipEventRecord(ev[1], s));
@@ -1010,10 +1015,12 @@ struct Engine {
       if (n <= 0) continue;
       nq += n;
       GradLaunch a{tasks_p + bval[cp], n, pairs_d.p, ppos_d.p, pk_d.p, pa_d.p, &ra, Pj, Pk, Pk2, nbf,
-                   sh_atom_d.p, natoms, kscale, grad_d.p, grad_d.p + 3 * natoms, sph_d.p};
+                   sh_atom_d.p, natoms, kscale, grad_d.p, grad_d.p + 3 * natoms, kGradCopies, sph_d.p};
       launch_grad(cp_bra[cp], cp_ket[cp], basis.pure, a, s);
       HIP_CHECK(hipGetLastError());
     }
+    launch_fold_copies(grad_d.p, 6 * natoms, kGradCopies, s);
+    HIP_CHECK(hipGetLastError());
     HIP_CHECK(hipEventRecord(ev[2], s));
     std::vector<double> g(6 * (size_t)natoms);
     HIP_CHECK(hipMemcpyAsync(g.data(), grad_d.p, sizeof(double) * g.size(), hipMemcpyDeviceToHost, s));

@@ -205,10 +205,14 @@ QFE_DI void grad_task(int2 tk, const PairHdr* __restrict__ pairs, const double4*
   }
 }
 
+// Blocks of the gradient kernels of one launch: eight times the CUs
+constexpr int kGradBlocks = 2048;
+
 // One thread per canonical task; bra cartesians [Q0, Q1) and ket cartesians
 // [K0, K1) of the class (the chunks keep every instance free of register
 // spills).  With lds the block sums its contributions in LDS ([2][3][natoms])
 // and flushes one atomic per entry; otherwise each thread adds to global.
+// Blocks add to one of ncopy copies of the gradient (a power of two).
 template <class C, int Q0, int Q1, int K0, int K1>
 __global__ __launch_bounds__(256) void k_eri_grad(const int2* __restrict__ tasks, long long ntask,
                                                   const PairHdr* __restrict__ pairs,
@@ -217,14 +221,17 @@ __global__ __launch_bounds__(256) void k_eri_grad(const int2* __restrict__ tasks
                                                   const double* __restrict__ P, const double* __restrict__ Pk,
                                                   const double* __restrict__ Pk2, int nbf,
                                                   const int* __restrict__ sh_atom, int natoms, double kscale,
-                                                  int lds, double* __restrict__ gJ, double* __restrict__ gK) {
+                                                  int lds, int ncopy, double* __restrict__ gJ,
+                                                  double* __restrict__ gK) {
   extern __shared__ double sg[];
+  gJ += (size_t)(blockIdx.x & (unsigned)(ncopy - 1)) * 6 * natoms;
+  gK += (size_t)(blockIdx.x & (unsigned)(ncopy - 1)) * 6 * natoms;
   if (lds) {
     for (int i = threadIdx.x; i < 6 * natoms; i += blockDim.x) sg[i] = 0.0;
     __syncthreads();
   }
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < ntask) {
+  for (long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x; t < ntask;
+       t += (long long)gridDim.x * blockDim.x) {
     const int2 tk = tasks[t];
     double gj[3][3], gk[3][3];
     grad_task<C, Q0, Q1, K0, K1>(tk, pairs, ppos, pk, pa, ra, P, Pk, Pk2, nbf, kscale, gj, gk);
@@ -266,7 +273,10 @@ struct GradOps {
     static_assert(C0 < C1 && C1 <= NCH && (!LAST || C1 == NCH), "chunk range does not match the class");
     if (a.ntask <= 0) return;
     const int block = 256;
-    const long long grid = (a.ntask + block - 1) / block;
+    // at most kGradBlocks blocks, each over several tasks a thread: a block
+    // flushes up to 6 sums an atom, and those atomics, not the integrals,
+    // bounded the light classes with a block for every 256 tasks
+    const long long grid = std::min((a.ntask + block - 1) / block, (long long)kGradBlocks);
     const int lds = a.natoms * 6 * (int)sizeof(double) <= 64 * 1024 ? 1 : 0;
     const size_t shm = lds ? (size_t)a.natoms * 6 * sizeof(double) : 0;
     hsfor<C1 - C0>([&](auto cc) {
@@ -276,7 +286,7 @@ struct GradOps {
       constexpr int k0 = k * K::KCH, k1 = (k0 + K::KCH < C::NKETC) ? k0 + K::KCH : C::NKETC;
       hipLaunchKernelGGL((k_eri_grad<C, q0, q1, k0, k1>), dim3((unsigned)grid), dim3(block), shm, s, a.tasks,
                          a.ntask, a.pairs, a.ppos, a.pk, a.pa, *a.ra, a.P, a.Pk, a.Pk2, a.nbf, a.sh_atom, a.natoms, a.kscale,
-                         lds, a.gJ, a.gK);
+                         lds, a.ncopy, a.gJ, a.gK);
     });
   }
 };

@@ -17,6 +17,7 @@
 #pragma once
 
 #include "eri_coop.hpp"
+#include "eri_grad.hpp"
 
 namespace qfe {
 
@@ -50,7 +51,9 @@ __global__ __launch_bounds__(G::BLK) void k_eri_grad_coop(
     const double4* __restrict__ ppos, const double* __restrict__ pk, const double* __restrict__ pa, RysArgs ra,
     const double* __restrict__ sph, const double* __restrict__ P, const double* __restrict__ Pk,
     const double* __restrict__ Pk2, int nbf, const int* __restrict__ sh_atom, int natoms, double kscale,
-    double* __restrict__ gJ, double* __restrict__ gK) {
+    int ncopy, double* __restrict__ gJ, double* __restrict__ gK) {
+  gJ += (size_t)(blockIdx.x & (unsigned)(ncopy - 1)) * 6 * natoms;
+  gK += (size_t)(blockIdx.x & (unsigned)(ncopy - 1)) * 6 * natoms;
   constexpr double TWO_PI_52 = 34.98683665524972;
   __shared__ double tab[G::CM * 3 * G::NI];
   __shared__ double par[G::CM * 3];
@@ -217,7 +220,8 @@ void grad_coop(const GradLaunch& a, hipStream_t s) {
   if (a.sph == nullptr) throw std::runtime_error("solid-harmonic table missing for the cooperative gradient kernel");
   const long long grid = std::min(a.ntask, 65536LL);
   hipLaunchKernelGGL((k_eri_grad_coop<G>), dim3((unsigned)grid), dim3(G::BLK), 0, s, a.tasks, a.ntask, a.pairs, a.ppos,
-                     a.pk, a.pa, *a.ra, a.sph, a.P, a.Pk, a.Pk2, a.nbf, a.sh_atom, a.natoms, a.kscale, a.gJ, a.gK);
+                     a.pk, a.pa, *a.ra, a.sph, a.P, a.Pk, a.Pk2, a.nbf, a.sh_atom, a.natoms, a.kscale,
+                     a.ncopy, a.gJ, a.gK);
 }
 
 }  // namespace qfe

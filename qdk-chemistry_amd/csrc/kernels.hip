@@ -538,6 +538,20 @@ void launch_jcd_tiles(const int4* tiles, int ntiles, int nk, int nsb, const int*
   }
 }
 
+// ------------------------------------------------------------ gradient copies
+__global__ __launch_bounds__(256) void k_fold_copies(double* __restrict__ g, int n, int ncopy) {
+  const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  if (i >= n) return;
+  double v = g[i];
+  for (int c = 1; c < ncopy; ++c) v += g[(size_t)c * n + i];
+  g[i] = v;
+}
+
+void launch_fold_copies(double* g, int n, int ncopy, hipStream_t s) {
+  if (n <= 0 || ncopy <= 1) return;
+  hipLaunchKernelGGL(k_fold_copies, dim3((n + 255) / 256), dim3(256), 0, s, g, n, ncopy);
+}
+
 __global__ __launch_bounds__(256) void k_copy_words(const unsigned long long* __restrict__ src,
                                                     unsigned long long* __restrict__ dst, size_t n) {
   const size_t stride = (size_t)gridDim.x * blockDim.x;

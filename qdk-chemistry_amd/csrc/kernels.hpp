@@ -94,8 +94,9 @@ struct GradLaunch {
   const int* sh_atom;
   int natoms;
   double kscale;
-  double* gJ;             // 3 * natoms, xyz-major
+  double* gJ;             // 3 * natoms, xyz-major: copy 0 of ncopy, 6 * natoms apart
   double* gK;
+  int ncopy;              // copies of (gJ, gK) that the blocks spread their atomics over (a power of two)
   const double* sph;      // device copy of the solid-harmonic table kSph (cooperative kernels)
 };
 

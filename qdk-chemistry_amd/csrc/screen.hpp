@@ -75,6 +75,8 @@ void launch_jcd_tiles(const int4* tiles, int ntiles, int nk, int nsb, const int*
 // build, symmetrised: J = (Jx + Jx^T) / 4, K = kq (Kx + Kx^T) / 2
 void launch_fixed_finish(const unsigned long long* Jx, const unsigned long long* Kx, double* J, double* K, int n,
                          double kq, hipStream_t s);
+// g[i] = sum of its ncopy copies, n apart (the gradient's accumulators)
+void launch_fold_copies(double* g, int n, int ncopy, hipStream_t s);
 // Profiling: add to *count the primitive quartets that the class kernels
 // evaluate for the tasks [0, ntask): the same prefix walk over primitives
 // sorted by sig, in the same precision and with the same cut, without the
