@@ -1010,14 +1010,35 @@ struct Engine {
     HIP_CHECK(hipEventRecord(ev[1], s));
     const int ncp = (int)cp_bra.size();
     long long nq = 0;
+    // the classes are independent (their contributions are added with
+    // atomics): spread over the streams by work like those of a J/K build
+    const int nst = 1 + (int)side.size();
+    std::vector<std::pair<double, int>> jobs;  // (quartets x functions per quartet, class pair)
     for (int cp = 0; cp < ncp; ++cp) {
       const long long n = bval[cp + 1] - bval[cp];
       if (n <= 0) continue;
       nq += n;
-      GradLaunch a{tasks_p + bval[cp], n, pairs_d.p, ppos_d.p, pk_d.p, pa_d.p, &ra, Pj, Pk, Pk2, nbf,
-                   sh_atom_d.p, natoms, kscale, grad_d.p, grad_d.p + 3 * natoms, kGradCopies, sph_d.p};
-      launch_grad(cp_bra[cp], cp_ket[cp], basis.pure, a, s);
+      jobs.push_back({(double)n * nfun_pair_class(cp_bra[cp]) * nfun_pair_class(cp_ket[cp]), cp});
+    }
+    if (nst > 1) {
+      std::stable_sort(jobs.begin(), jobs.end(), [](const auto& x, const auto& y) { return x.first > y.first; });
+      HIP_CHECK(hipEventRecord(fork_ev, s));
+      for (hipStream_t st : side) HIP_CHECK(hipStreamWaitEvent(st, fork_ev, 0));
+    }
+    std::vector<double> load(nst, 0.0);
+    for (const auto& job : jobs) {
+      const int cp = job.second;
+      const int k = (int)(std::min_element(load.begin(), load.end()) - load.begin());
+      load[k] += job.first;
+      hipStream_t cs = k == 0 ? s : side[k - 1];
+      GradLaunch a{tasks_p + bval[cp], bval[cp + 1] - bval[cp], pairs_d.p, ppos_d.p, pk_d.p, pa_d.p, &ra, Pj, Pk,
+                   Pk2, nbf, sh_atom_d.p, natoms, kscale, grad_d.p, grad_d.p + 3 * natoms, kGradCopies, sph_d.p};
+      launch_grad(cp_bra[cp], cp_ket[cp], basis.pure, a, cs);
       HIP_CHECK(hipGetLastError());
+    }
+    for (int k = 1; k < nst; ++k) {
+      HIP_CHECK(hipEventRecord(side_ev[k - 1], side[k - 1]));
+      HIP_CHECK(hipStreamWaitEvent(s, side_ev[k - 1], 0));
     }
     launch_fold_copies(grad_d.p, 6 * natoms, kGradCopies, s);
     HIP_CHECK(hipGetLastError());
