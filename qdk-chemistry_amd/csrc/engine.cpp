@@ -275,7 +275,7 @@ struct Engine {
   DevBuf<int> cp_nk_d;
   DevBuf<int4> jtiles_d;
   struct JTileGroup {
-    int nk, nsb, begin, count;
+    int nk, nsb, begin, count, tket;  // tket: ket positions per tile
   };
   std::vector<JTileGroup> jt_groups;
   long long jslot_total = 0;
@@ -732,6 +732,7 @@ struct Engine {
     std::vector<int> cp_nk(ncp);
     for (int cp = 0; cp < ncp; ++cp) cp_nk[cp] = nfun_pair_class(cp_ket[cp]);
     cp_nk_d.upload(cp_nk, stream);
+    // (bra bucket, ket bucket) blocks {first item, stride, bra bucket, ket bucket} by ket pair size
     std::map<int, std::vector<int4>> by_nk;
     std::map<int, int> nsb_of;
     for (int cp = 0; cp < ncp; ++cp) {
@@ -745,9 +746,7 @@ struct Engine {
       const int nk = cp_nk[cp];
       nsb_of[nk] = nsph(lb, true);
       std::vector<int4>& out = by_nk[nk];
-      for (int kb = kbf; kb < kbl; ++kb) {
-        const int2 kbk = buckets_h[kb];
-        const int ksize = kbk.y - kbk.x;
+      for (int kb = kbf; kb < kbl; ++kb)
         for (int bb = std::max(bbf, kb); bb < bbl; ++bb) {
           const int2 bbk = buckets_h[bb];
           const int stride = (cb == ck) ? bb - kbf + 1 : kbl - kbf;
@@ -760,21 +759,36 @@ struct Engine {
             const int2 it = items_h[item0 + (p - bbk.x) * stride];
             if (it.x != p || it.y != kb) throw std::runtime_error("J_cd tile layout does not match the work items");
           }
-          for (int p0 = bbk.x; p0 < bbk.y; p0 += kJcdTileBra) {
-            const int np = std::min(kJcdTileBra, bbk.y - p0);
-            // same bucket: bra pair p holds positions j <= p - first pair only
-            const int jmax = (bb == kb) ? std::min(ksize, p0 + np - kbk.x) : ksize;
-            for (int j0 = 0; j0 < jmax; j0 += kJcdTileKet)
-              out.push_back(make_int4(item0 + (p0 - bbk.x) * stride, (stride << 16) | np, kbk.x, j0));
-          }
+          out.push_back(make_int4(item0, stride, bb, kb));
         }
-      }
     }
+    // Tiles of tbra bra pairs x tket positions, cut until a group has
+    // kJcdTilesMin of them: one wave walks a tile, so a small system's few
+    // large tiles left most of the GPU idle behind one long chain each
+    // ((H2O)16/cc-pVDZ: 12 to 432 waves a group, 5.2 ms over all groups
+    // with 256 x 1024 tiles).  Large systems keep large tiles: a tile ends
+    // with one atomic per position and function.
     std::vector<int4> all;
     jt_groups.clear();
     for (auto& kv : by_nk) {
-      jt_groups.push_back({kv.first, nsb_of[kv.first], (int)all.size(), (int)kv.second.size()});
-      all.insert(all.end(), kv.second.begin(), kv.second.end());
+      const int begin = (int)all.size();
+      int tket = kJcdTileKet;
+      for (int tbra = kJcdTileBra;; tket > 64 ? tket /= 2 : tbra /= 2) {
+        all.resize(begin);
+        for (const int4& r : kv.second) {
+          const int2 bbk = buckets_h[r.z], kbk = buckets_h[r.w];
+          const int ksize = kbk.y - kbk.x;
+          for (int p0 = bbk.x; p0 < bbk.y; p0 += tbra) {
+            const int np = std::min(tbra, bbk.y - p0);
+            // same bucket: bra pair p holds positions j <= p - first pair only
+            const int jmax = (r.z == r.w) ? std::min(ksize, p0 + np - kbk.x) : ksize;
+            for (int j0 = 0; j0 < jmax; j0 += tket)
+              all.push_back(make_int4(r.x + (p0 - bbk.x) * r.y, (r.y << 16) | np, kbk.x, j0));
+          }
+        }
+        if ((int)all.size() - begin >= kJcdTilesMin || (tket <= 64 && tbra <= 32)) break;
+      }
+      jt_groups.push_back({kv.first, nsb_of[kv.first], begin, (int)all.size() - begin, tket});
     }
     jtiles_d.upload(all, stream);
   }
@@ -1136,7 +1150,7 @@ struct Engine {
             if (nfun_pair_class(cp_ket[job.cp]) == g.nk)
               HIP_CHECK(hipStreamWaitEvent(gs, done_ev[(size_t)job.prec * ncp + job.cp], 0));
         }
-        launch_jcd_tiles(jtiles_d.p + g.begin, g.count, g.nk, g.nsb, nslot_d.p, jslot_d.p, mbase_d.p, jmask_p,
+        launch_jcd_tiles(jtiles_d.p + g.begin, g.count, g.tket, g.nk, g.nsb, nslot_d.p, jslot_d.p, mbase_d.p, jmask_p,
                          jbuf_p, pairs_d.p, Jd, nbf, Jx, fxo_d.p, gs);
         HIP_CHECK(hipGetLastError());
       }

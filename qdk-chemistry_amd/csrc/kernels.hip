@@ -393,7 +393,7 @@ void launch_fixed_finish(const unsigned long long* Jx, const unsigned long long*
 // Share slots: item (p, kb) owns nslot[item] / NK positions j (ket pair
 // q = first pair of bucket kb + j), NK doubles each, from jbuf + jslot[item].
 // A tile is up to 256 consecutive bra pairs of one bra bucket (items
-// item0 + i * stride, i < np) against positions [j0, j0 + kJcdTileKet) of one
+// item0 + i * stride, i < np) against positions [j0, j0 + tket) of one
 // ket bucket whose first pair is q0.  One wave per tile walks the tile's
 // items (their prefix lengths, slot bases and mask bases are loaded once, four
 // per lane); for each 64-position block it gathers every item's survivor word
@@ -402,7 +402,7 @@ void launch_fixed_finish(const unsigned long long* Jx, const unsigned long long*
 // block as contiguous runs (lane l holds elements l, l + 64, ... of the
 // block's 64 * NK doubles) and adds the sums to J.
 template <int NK>
-__global__ __launch_bounds__(256) void k_jcd_tiles(const int4* __restrict__ tiles, int ntiles,
+__global__ __launch_bounds__(256) void k_jcd_tiles(const int4* __restrict__ tiles, int ntiles, int tket,
                                                    const int* __restrict__ nslot,
                                                    const long long* __restrict__ jslot,
                                                    const long long* __restrict__ mbase,
@@ -438,7 +438,7 @@ __global__ __launch_bounds__(256) void k_jcd_tiles(const int4* __restrict__ tile
     const int v = __shfl_xor(nmax, o);
     nmax = v > nmax ? v : nmax;
   }
-  const int jend = tl.w + kJcdTileKet < nmax ? tl.w + kJcdTileKet : nmax;
+  const int jend = tl.w + tket < nmax ? tl.w + tket : nmax;
   // lanes own flattened elements of the 64-position block: element
   // e = f * 64 + lane is function e % NK of position jc + e / NK, so a wave's
   // share loads are contiguous 512-byte runs of the item's slots
@@ -510,30 +510,30 @@ __global__ __launch_bounds__(256) void k_jcd_tiles(const int4* __restrict__ tile
 }
 
 template <int NK>
-static void jcd_tiles_launch(const int4* tiles, int ntiles, const int* nslot, const long long* jslot,
+static void jcd_tiles_launch(const int4* tiles, int ntiles, int tket, const int* nslot, const long long* jslot,
                              const long long* mbase, const unsigned long long* jmask, const double* jbuf,
                              const PairHdr* pairs, int nsb, double* J, int nbf, unsigned long long* Jx, int* over,
                              hipStream_t s) {
   const long long threads = (long long)ntiles * 64;
-  hipLaunchKernelGGL((k_jcd_tiles<NK>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, tiles, ntiles,
+  hipLaunchKernelGGL((k_jcd_tiles<NK>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, tiles, ntiles, tket,
                      nslot, jslot, mbase, jmask, jbuf, pairs, nsb, J, nbf, Jx, over);
 }
 
-void launch_jcd_tiles(const int4* tiles, int ntiles, int nk, int nsb, const int* nslot, const long long* jslot,
+void launch_jcd_tiles(const int4* tiles, int ntiles, int tket, int nk, int nsb, const int* nslot, const long long* jslot,
                       const long long* mbase, const unsigned long long* jmask, const double* jbuf,
                       const PairHdr* pairs, double* J, int nbf, unsigned long long* Jx, int* over, hipStream_t s) {
   if (ntiles <= 0) return;
   switch (nk) {
-    case 1: jcd_tiles_launch<1>(tiles, ntiles, nslot, jslot, mbase, jmask, jbuf, pairs, nsb, J, nbf, Jx, over, s); break;
-    case 3: jcd_tiles_launch<3>(tiles, ntiles, nslot, jslot, mbase, jmask, jbuf, pairs, nsb, J, nbf, Jx, over, s); break;
-    case 5: jcd_tiles_launch<5>(tiles, ntiles, nslot, jslot, mbase, jmask, jbuf, pairs, nsb, J, nbf, Jx, over, s); break;
-    case 7: jcd_tiles_launch<7>(tiles, ntiles, nslot, jslot, mbase, jmask, jbuf, pairs, nsb, J, nbf, Jx, over, s); break;
-    case 9: jcd_tiles_launch<9>(tiles, ntiles, nslot, jslot, mbase, jmask, jbuf, pairs, nsb, J, nbf, Jx, over, s); break;
-    case 15: jcd_tiles_launch<15>(tiles, ntiles, nslot, jslot, mbase, jmask, jbuf, pairs, nsb, J, nbf, Jx, over, s); break;
-    case 21: jcd_tiles_launch<21>(tiles, ntiles, nslot, jslot, mbase, jmask, jbuf, pairs, nsb, J, nbf, Jx, over, s); break;
-    case 25: jcd_tiles_launch<25>(tiles, ntiles, nslot, jslot, mbase, jmask, jbuf, pairs, nsb, J, nbf, Jx, over, s); break;
-    case 35: jcd_tiles_launch<35>(tiles, ntiles, nslot, jslot, mbase, jmask, jbuf, pairs, nsb, J, nbf, Jx, over, s); break;
-    case 49: jcd_tiles_launch<49>(tiles, ntiles, nslot, jslot, mbase, jmask, jbuf, pairs, nsb, J, nbf, Jx, over, s); break;
+    case 1: jcd_tiles_launch<1>(tiles, ntiles, tket, nslot, jslot, mbase, jmask, jbuf, pairs, nsb, J, nbf, Jx, over, s); break;
+    case 3: jcd_tiles_launch<3>(tiles, ntiles, tket, nslot, jslot, mbase, jmask, jbuf, pairs, nsb, J, nbf, Jx, over, s); break;
+    case 5: jcd_tiles_launch<5>(tiles, ntiles, tket, nslot, jslot, mbase, jmask, jbuf, pairs, nsb, J, nbf, Jx, over, s); break;
+    case 7: jcd_tiles_launch<7>(tiles, ntiles, tket, nslot, jslot, mbase, jmask, jbuf, pairs, nsb, J, nbf, Jx, over, s); break;
+    case 9: jcd_tiles_launch<9>(tiles, ntiles, tket, nslot, jslot, mbase, jmask, jbuf, pairs, nsb, J, nbf, Jx, over, s); break;
+    case 15: jcd_tiles_launch<15>(tiles, ntiles, tket, nslot, jslot, mbase, jmask, jbuf, pairs, nsb, J, nbf, Jx, over, s); break;
+    case 21: jcd_tiles_launch<21>(tiles, ntiles, tket, nslot, jslot, mbase, jmask, jbuf, pairs, nsb, J, nbf, Jx, over, s); break;
+    case 25: jcd_tiles_launch<25>(tiles, ntiles, tket, nslot, jslot, mbase, jmask, jbuf, pairs, nsb, J, nbf, Jx, over, s); break;
+    case 35: jcd_tiles_launch<35>(tiles, ntiles, tket, nslot, jslot, mbase, jmask, jbuf, pairs, nsb, J, nbf, Jx, over, s); break;
+    case 49: jcd_tiles_launch<49>(tiles, ntiles, tket, nslot, jslot, mbase, jmask, jbuf, pairs, nsb, J, nbf, Jx, over, s); break;
     default: break;  // no other pure pair sizes up to f
   }
 }

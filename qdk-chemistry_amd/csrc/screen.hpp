@@ -66,9 +66,10 @@ void launch_symmetrize(double* J, double* K, int n, hipStream_t s);
 // shares of the surviving quartets.  launch_jcd_tiles sums them per ket pair
 // into J for the tiles of one ket pair size nk (nsb = functions of the pair's
 // second shell); a tile is int4 {first item, stride << 16 | bra pairs
-// (<= 256), first pair of the ket bucket, first position (a multiple of 64)}.
+// (<= 256), first pair of the ket bucket, first position (a multiple of 64)}
+// and covers tket positions.
 // (Jx non-null: the sums go to the fixed-point pairs of a deterministic build)
-void launch_jcd_tiles(const int4* tiles, int ntiles, int nk, int nsb, const int* nslot, const long long* jslot,
+void launch_jcd_tiles(const int4* tiles, int ntiles, int tket, int nk, int nsb, const int* nslot, const long long* jslot,
                       const long long* mbase, const unsigned long long* jmask, const double* jbuf,
                       const PairHdr* pairs, double* J, int nbf, unsigned long long* Jx, int* over, hipStream_t s);
 // J, K (either may be null) from the fixed-point sums of a deterministic
@@ -84,8 +85,9 @@ void launch_fold_copies(double* g, int n, int ncopy, hipStream_t s);
 void launch_count_prims(const int2* tasks, long long ntask, const PairHdr* pairs, const double* sig,
                         const float* sig32, const double* pmax, int prim_screen, int fp32,
                         unsigned long long* count, hipStream_t s);
-constexpr int kJcdTileBra = 256;   // bra pairs per tile
-constexpr int kJcdTileKet = 1024;  // ket positions per tile
+constexpr int kJcdTileBra = 256;   // bra pairs per tile, at most
+constexpr int kJcdTileKet = 1024;  // ket positions per tile, at most (a multiple of 64)
+constexpr int kJcdTilesMin = 4096;  // tiles of one ket pair size below which they are cut smaller
 
 // plain device-to-device copy of n 8-byte words (also the reference kernel for
 // HBM traffic counters: it moves exactly 8n bytes each way)
