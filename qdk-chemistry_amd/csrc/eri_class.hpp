@@ -248,7 +248,7 @@ __global__ __launch_bounds__(BLK) void k_eri_jk_seg(const int2* __restrict__ seg
     jij[qq] = 0.0;
   });
   const double dbra = bra.sa == bra.sb ? 1.0 : 2.0;
-  for (long long t = t0 + threadIdx.x; t < t1; t += blockDim.x) {
+  for (long long t = t1 - 1 - (long long)threadIdx.x; t >= t0; t -= blockDim.x) {
     const int2 tk = tasks[t];
     // classes with an f shell are bound by their integrals, not by this
     // load: they read the full header (the compact record costs them registers)
