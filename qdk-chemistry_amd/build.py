@@ -48,19 +48,15 @@ def _nsph(l):
 
 
 # Accumulators per thread of classes whose kernels spilled with the default
-# (48 up to d shells; with an f shell 24, and 16 from L = 11 on): the class's
-# generated sources define QFE_JK_ACC_F, which JKChunks (csrc/eri_class.hpp)
-# then uses.  (ff|dd) at 18 keeps its 98 chunks (two ket halves of 18
-# cartesians instead of 24 + 12).
-JK_ACC_F = {(3, 3, 3, 2): 12, (3, 3, 2, 2): 18, (2, 1, 1, 1): 40}
+# (48 up to d shells; with an f shell 24): the class's generated sources define
+# QFE_JK_ACC_F, which JKChunks (csrc/eri_class.hpp) then uses.
+JK_ACC_F = {(2, 1, 1, 1): 40}
 
 
 def jk_acc(la, lb, lc, ld):
     if (la, lb, lc, ld) in JK_ACC_F:
         return JK_ACC_F[(la, lb, lc, ld)]
-    if max(la, lb, lc, ld) <= 2:
-        return 48
-    return 16 if la + lb + lc + ld >= 11 else 24
+    return 48 if max(la, lb, lc, ld) <= 2 else 24
 
 
 def jk_chunks(la, lb, lc, ld):
@@ -86,11 +82,22 @@ def jk_chunks(la, lb, lc, ld):
     return min(nsa * mp, nbu) * nkch
 
 
-def schwarz_block(la, lb):
-    """Doubles of the Schwarz staging block per pair (classes with f shells)."""
-    if max(la, lb) <= 2:
-        return 0
-    return _nsph(la) * _nsph(lb) * _ncart(la) * _ncart(lb)
+def jk_segment(la, lb, lc, ld):
+    """Whether a class has segment kernels (csrc/eri_class.hpp).  Every chunk of
+    a class is a launch that repeats its integrals; from eight chunks on, the
+    f-shell classes are faster in the cooperative kernel (csrc/eri_jk_coop.hpp)
+    at every size measured: (ff|ff) in 343 chunks 9.4 ms against 36 us for 167
+    quartets, (fd|dp) 35 chunks 2.5 against 1.8 ms for 114,826."""
+    return max(la, lb, lc, ld) <= 2 or jk_chunks(la, lb, lc, ld) <= 7
+
+
+def jk_coop_tasks(la, lb, lc, ld):
+    """Quartets up to which a class with segment kernels runs in the cooperative
+    kernel.  A segment kernel takes 0.1-1 ms however few quartets there are (a
+    thread's chain of primitive quartets, once per chunk); the cooperative one
+    takes 3-15 ns a quartet, more than a full segment kernel."""
+    return (50000 if jk_chunks(la, lb, lc, ld) >= 3 or (la, lb, lc, ld) == (1, 1, 1, 1)
+            else 25000 if la + lb + lc + ld <= 1 else 15000)
 
 
 # highest l of the gradient kernels
@@ -134,7 +141,7 @@ def gen_sources():
     os.makedirs(GEN, exist_ok=True)
     pcs = pair_classes(MAX_L)
     files = []
-    decls, jk_cases, sw_cases, gr_cases, sb_cases = [], [], [], [], []
+    decls, jk_cases, sw_cases, gr_cases = [], [], [], []
     head = ["// generated by build.py", '#include "../../eri_grad.hpp"', "namespace qfe {"]
     for b, (la, lb) in enumerate(pcs):
         for k, (lc, ld) in enumerate(pcs[: b + 1]):
@@ -144,9 +151,10 @@ def gen_sources():
             ltot = la + lb + lc + ld
             nch = jk_chunks(la, lb, lc, ld)
             # ERI J/K (+ Schwarz on the diagonal): kernels per chunk
+            seg = jk_segment(la, lb, lc, ld)
             kpc = (1 if fcls else 4) + (1 if b == k else 0)  # segment kernels (+ Schwarz)
             jk_calls, sw_calls = [], []
-            parts = _parts(nch, kpc, ltot)
+            parts = _parts(nch, kpc, ltot) if seg else []
             for i, (c0, c1) in enumerate(parts):
                 last = "true" if c1 == nch else "false"
                 sfx = f"_p{i}" if len(parts) > 1 else ""
@@ -156,22 +164,34 @@ def gen_sources():
                                f"{ops}::{fn}<{c0}, {c1}, {last}>(a, s); }}"]
                 decls.append(f"void jk_cls_{tag}{sfx}(const JKLaunch& a, hipStream_t s);")
                 jk_calls.append(f"jk_cls_{tag}{sfx}(a, s);")
-                if b == k:
+                if b == k and not fcls:
                     body.append(f"void schwarz_cls_{tag}{sfx}(const SchwarzLaunch& a, hipStream_t s) {{ "
                                 f"{ops}::schwarz_range<{c0}, {c1}, {last}>(a, s); }}")
                     decls.append(f"void schwarz_cls_{tag}{sfx}(const SchwarzLaunch& a, hipStream_t s);")
                     sw_calls.append(f"schwarz_cls_{tag}{sfx}(a, s);")
-                    if i == 0:
-                        body.append(f"void schwarz_fold_cls_{tag}(const SchwarzLaunch& a, hipStream_t s) {{ "
-                                    f"{ops}::schwarz_fold(a, s); }}")
-                        decls.append(f"void schwarz_fold_cls_{tag}(const SchwarzLaunch& a, hipStream_t s);")
                 path = os.path.join(GEN, f"cls_{tag}{sfx}.hip")
                 _write_if_changed(path, "\n".join(body + ["}  // namespace qfe"]) + "\n")
                 files.append(path)
-            jk_cases.append(f"  if (cb == {b} && ck == {k}) {{ {' '.join(jk_calls)} return; }}")
+            # the cooperative J/K kernel (a block per quartet), and the
+            # Schwarz kernel of the f-shell classes
+            body = ["// generated by build.py", '#include "../../eri_jk_coop.hpp"', "namespace qfe {",
+                    f"void jkc_cls_{tag}(const JKLaunch& a, hipStream_t s) {{ "
+                    f"jk_coop<{la}, {lb}, {lc}, {ld}>(a, s); }}"]
+            decls.append(f"void jkc_cls_{tag}(const JKLaunch& a, hipStream_t s);")
+            if b == k and fcls:
+                body.append(f"void schwarz_cls_{tag}(const SchwarzLaunch& a, hipStream_t s) {{ "
+                            f"schwarz_coop<{la}, {lb}>(a, s); }}")
+                decls.append(f"void schwarz_cls_{tag}(const SchwarzLaunch& a, hipStream_t s);")
+                sw_calls.append(f"schwarz_cls_{tag}(a, s);")
+            path = os.path.join(GEN, f"jkc_{tag}.hip")
+            _write_if_changed(path, "\n".join(body + ["}  // namespace qfe"]) + "\n")
+            files.append(path)
+            few = f" && a.coop && a.ntask <= {jk_coop_tasks(la, lb, lc, ld)}" if seg else ""
+            jk_cases.append(f"  if (cb == {b} && ck == {k}{few}) {{ jkc_cls_{tag}(a, s); return; }}")
+            if seg:
+                jk_cases.append(f"  if (cb == {b} && ck == {k}) {{ {' '.join(jk_calls)} return; }}")
             if b == k:
-                sw_cases.append(f"  if (c == {b}) {{ {' '.join(sw_calls)} schwarz_fold_cls_{tag}(a, s); return; }}")
-                sb_cases.append(f"  if (c == {b}) return {schwarz_block(la, lb)};")
+                sw_cases.append(f"  if (c == {b}) {{ {' '.join(sw_calls)} return; }}")
             # cooperative gradient kernel (a block per quartet): every class with
             # an f shell, the others up to grad_coop_tasks quartets
             body = ["// generated by build.py", '#include "../../eri_grad_coop.hpp"', "namespace qfe {",
@@ -208,7 +228,6 @@ def gen_sources():
         "void launch_schwarz(int c, bool pure, const SchwarzLaunch& a, hipStream_t s) {",
         '  if (!pure) throw std::runtime_error("cartesian bases are not compiled");'] + sw_cases + [
         '  throw std::runtime_error("Schwarz class not compiled");', "}",
-        "int schwarz_block(int c) {"] + sb_cases + ["  return 0;", "}",
         "void launch_grad(int cb, int ck, bool pure, const GradLaunch& a, hipStream_t s) {",
         '  if (!pure) throw std::runtime_error("cartesian bases are not compiled");'] + gr_cases + [
         '  throw std::runtime_error("gradient class not compiled");', "}",
@@ -231,6 +250,11 @@ def gen_sources():
              "    }", "  });", "  return K::NCH;", "}", "}  // namespace qfe",
              f'{extern}int {fname}(int la, int lb, int lc, int ld, int cap, int* out) {{']
         for (la, lb, lc, ld) in classes:
+            if not jk_segment(la, lb, lc, ld):  # one cooperative kernel for the whole quartet
+                t.append(f"  if (la == {la} && lb == {lb} && lc == {lc} && ld == {ld}) {{ if (cap > 0) {{ out[0] = "
+                         f"out[2] = 0; out[1] = {_nsph(la) * _nsph(lb)}; out[3] = {_ncart(lc) * _ncart(ld)}; }} "
+                         f"return 1; }}")
+                continue
             t.append(f"  if (la == {la} && lb == {lb} && lc == {lc} && ld == {ld}) "
                      f"return qfe::chunk_table<qfe::ClassOps<{la}, {lb}, {lc}, {ld}, true>>(cap, out);")
         return t + ["  return -1;", "}"]
@@ -279,6 +303,8 @@ def _deps(src):
         hs = ["kernels.hpp"]
     elif name.startswith("chunks"):
         hs = core + ["eri_class.hpp"]
+    elif name.startswith("jkc_"):
+        hs = core + ["fixed_point.hpp", "eri_class.hpp", "eri_coop.hpp", "eri_jk_coop.hpp"]
     elif name.startswith("gradc_"):
         hs = core + ["eri_class.hpp", "eri_grad.hpp", "eri_coop.hpp", "eri_grad_coop.hpp"]
     elif name.startswith("grad_") or name.startswith("cls_"):

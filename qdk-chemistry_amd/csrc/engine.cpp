@@ -263,6 +263,7 @@ struct Engine {
   DevBuf<int> fxo_d;                 // fixed-point range overflow flag
   // primitive-quartet screening at the engine precision (QFE_PRIM_SCREEN=0: off)
   bool prim_screen = true;
+  bool coop = true;                  // QFE_COOP=0: the segment kernels for every class that has them
   int kcol_tile = 0;                 // QFE_KCOL_TILE: cap on the exchange-row tile width
   std::vector<int> sh_bf0_h;         // first function of each shell (+ nbf), host
   std::vector<int> cls_pair_begin;  // first pair of each pair class (pairs are class-sorted)
@@ -524,23 +525,12 @@ struct Engine {
     std::vector<std::vector<int>> bycls(ncls);
     for (int i = 0; i < npair; ++i) bycls[hdr[i].cls].push_back(i);
     std::vector<DevBuf<int>> plist(ncls);
-    // f-shell classes stage their (ab|ab) blocks: batches of pairs that fit
-    // a staging buffer of at most kSchwarzStage doubles
-    constexpr size_t kSchwarzStage = (size_t)1 << 24;
-    DevBuf<double> stage;
     for (int c = 0; c < ncls; ++c) {
       if (bycls[c].empty()) continue;
       plist[c].upload(bycls[c], stream);
-      const int n = (int)bycls[c].size();
-      const size_t per = (size_t)schwarz_block(c);
-      const int batch = per ? (int)std::max<size_t>(1, std::min<size_t>((size_t)n, kSchwarzStage / per)) : n;
-      if (per) stage.alloc(per * (size_t)batch);
-      for (int i0 = 0; i0 < n; i0 += batch) {
-        SchwarzLaunch a{plist[c].p + i0, std::min(batch, n - i0), pairs_d.p, ppos_d.p, pk_d.p, &ra, q2.p,
-                        per ? stage.p : nullptr};
-        launch_schwarz(c, basis.pure, a, stream);
-        HIP_CHECK(hipGetLastError());
-      }
+      SchwarzLaunch a{plist[c].p, (int)bycls[c].size(), pairs_d.p, ppos_d.p, pk_d.p, &ra, q2.p};
+      launch_schwarz(c, basis.pure, a, stream);
+      HIP_CHECK(hipGetLastError());
     }
     std::vector<double> q2h(npair);
     HIP_CHECK(hipMemcpyAsync(q2h.data(), q2.p, sizeof(double) * npair, hipMemcpyDeviceToHost, stream));
@@ -833,6 +823,9 @@ struct Engine {
     // QFE_PRIM_SCREEN=0 evaluates every primitive quartet
     if (const char* e = std::getenv("QFE_PRIM_SCREEN"))
       if (e[0] == '0') prim_screen = false;
+    // QFE_COOP=0 runs the segment kernels also where a class has few quartets
+    if (const char* e = std::getenv("QFE_COOP"))
+      if (e[0] == '0') coop = false;
     // QFE_KCOL_TILE=<columns>: exchange-row tiles of at most that many
     // columns even where whole rows fit (exercises the tiled path)
     if (const char* e = std::getenv("QFE_KCOL_TILE")) kcol_tile = std::max(0, std::atoi(e));
@@ -1128,7 +1121,7 @@ struct Engine {
                    offsets_d.p + (prec ? (long long)items_h.size() : 0), tasks_p, lds_max,
                    jslots ? jbuf_p : nullptr, jslot_d.p, qpos_d.p, seg_min_waves,
                    pmax_d.p, prim_screen ? 1 : 0, det ? 1 : 0, Jx, Kx, fxo_d.p, sh_bf0_h.data(), nsh,
-                   kcol_tile, kets_d.p, shells_d.p};
+                   kcol_tile, kets_d.p, shells_d.p, coop ? 1 : 0, cls_pair_begin[cp_bra[cp]]};
         hipEvent_t* e = profile ? &cls_ev[4 * (size_t)cp + 2 * prec] : nullptr;
         if (e) HIP_CHECK(hipEventRecord(e[0], cs));
         launch_jk(cp_bra[cp], cp_ket[cp], basis.pure, a, cs);

@@ -50,8 +50,7 @@ constexpr int seg_bch(int hi) {
 
 // Accumulators per thread: bra functions x ket cartesians of one chunk.  48
 // for classes up to d shells (their whole ket block fits); classes with an f
-// shell hold fewer and are also chunked over the ket cartesians, so that no
-// kernel instance spills registers (24, and 16 from L = 11 on).
+// shell hold fewer (24), so that no kernel instance spills registers.
 constexpr int kAccMax = 48;
 // A class whose kernels spilled with the default is compiled with its own
 // QFE_JK_ACC_F (defined by its generated source).
@@ -61,7 +60,7 @@ constexpr int jk_acc() {
   return QFE_JK_ACC_F;
 #else
   if (C::LA <= 2 && C::LB <= 2 && C::LC <= 2 && C::LD <= 2) return kAccMax;
-  return C::L >= 11 ? 16 : 24;
+  return 24;
 #endif
 }
 template <class C>
@@ -405,48 +404,6 @@ __global__ __launch_bounds__(256) void k_schwarz(const int* __restrict__ plist, 
   unsafeAtomicAdd(&q2[p], s);
 }
 
-// Schwarz of classes with f shells, in two steps: each chunk kernel writes its
-// share (bra functions x ket cartesians) of the (ab|ab) block to blk, then the
-// fold transforms every bra function's ket row to output functions and adds
-// its sum of squares to q2 (the square needs the whole row, so it cannot be
-// taken per chunk).
-template <class C, int Q0, int Q1, int K0, int K1>
-__global__ __launch_bounds__(256) void k_schwarz_part(const int* __restrict__ plist, int npair,
-                                                      const PairHdr* __restrict__ pairs,
-                                                      const double4* __restrict__ ppos,
-                                                      const double* __restrict__ pk, RysArgs ra,
-                                                      double* __restrict__ blk) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= npair) return;
-  const PairHdr pr = pairs[plist[t]];
-  double acc[Q1 - Q0][K1 - K0];
-  contract_chunk<C, Q0, Q1, double, K0, K1>(pr, pr, ppos, pk, ra, acc);
-  sfor<Q1 - Q0>([&](auto qq) {
-    double* row = blk + ((size_t)t * C::NBRA + Q0 + qq) * C::NKETC + K0;
-    sfor<K1 - K0>([&](auto kk) { row[kk] = acc[qq][kk]; });
-  });
-}
-
-template <class C>
-__global__ __launch_bounds__(256) void k_schwarz_fold(const int* __restrict__ plist, int npair,
-                                                      const double* __restrict__ blk, double* __restrict__ q2) {
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (long long)npair * C::NBRA) return;
-  const double* row = blk + (size_t)i * C::NKETC;
-  double s = 0.0;
-  sfor<C::NSC>([&](auto mc) {
-    sfor<C::NSD>([&](auto md) {
-      double v = 0.0;
-      sfor<C::NKETC>([&](auto k) {
-        constexpr double c = sph_coef(C::LC, C::PURE, mc, k / C::NCD) * sph_coef(C::LD, C::PURE, md, k % C::NCD);
-        if constexpr (c != 0.0) v = fma(c, row[k], v);
-      });
-      s = fma(v, v, s);
-    });
-  });
-  unsafeAtomicAdd(&q2[plist[i / C::NBRA]], s);
-}
-
 // ------------------------------------------------------------ launchers
 template <int LA, int LB, int LC, int LD, bool PURE>
 struct ClassOps {
@@ -463,9 +420,6 @@ struct ClassOps {
       K::F ? 256
            : (C::L <= 1 ? 1024
                         : (C::L <= 3 ? ((C::L == 2 || C::FC == 0) ? 768 : 512) : (C::FC <= 1 ? 512 : 256)));
-  // doubles of the Schwarz staging block per pair (classes with f shells)
-  static constexpr int SCHWARZ_BLOCK = K::F ? C::NBRA * C::NKETC : 0;
-
   // dynamic LDS bytes of a segment block over W exchange columns: the K rows
   // (doubles, or fixed-point pairs in deterministic builds) and the P rows
   // with prow; seg_total adds the static J_ab slots
@@ -609,28 +563,14 @@ struct ClassOps {
   static void schwarz_range(const SchwarzLaunch& a, hipStream_t s) {
     static_assert(C0 < C1 && C1 <= NCH && (!LAST || C1 == NCH), "chunk range does not match the class");
     if (a.npair <= 0) return;
-    if (K::F && a.blk == nullptr) throw std::runtime_error("Schwarz staging block missing for an f-shell class");
+    static_assert(!K::F, "classes with f shells use schwarz_coop");
     const int block = 256;
     const int grid = (a.npair + block - 1) / block;
     hsfor<C1 - C0>([&](auto cc) {
       using A = typename K::template At<C0 + cc>;
-      if constexpr (K::F)
-        hipLaunchKernelGGL((k_schwarz_part<C, A::Q0, A::Q1, A::K0, A::K1>), dim3(grid), dim3(block), 0, s, a.plist,
-                           a.npair, a.pairs, a.ppos, a.pk, *a.ra, a.blk);
-      else
-        hipLaunchKernelGGL((k_schwarz<C, A::Q0, A::Q1>), dim3(grid), dim3(block), 0, s, a.plist, a.npair, a.pairs,
-                           a.ppos, a.pk, *a.ra, a.q2);
+      hipLaunchKernelGGL((k_schwarz<C, A::Q0, A::Q1>), dim3(grid), dim3(block), 0, s, a.plist, a.npair, a.pairs,
+                         a.ppos, a.pk, *a.ra, a.q2);
     });
-  }
-
-  // after every chunk range: fold the staged blocks (classes with f shells)
-  static void schwarz_fold(const SchwarzLaunch& a, hipStream_t s) {
-    if constexpr (K::F) {
-      if (a.npair <= 0) return;
-      const long long n = (long long)a.npair * C::NBRA;
-      hipLaunchKernelGGL((k_schwarz_fold<C>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a.plist, a.npair,
-                         a.blk, a.q2);
-    }
   }
 };
 

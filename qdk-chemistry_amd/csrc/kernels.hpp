@@ -77,6 +77,8 @@ struct JKLaunch {
   int kcol_tile;            // > 0: exchange-row tiles of at most this many columns (testing knob)
   const int4* kets;
   const double4* shells;
+  int coop;                 // 1: classes with few quartets run in the cooperative kernel
+  int bra0;                 // first pair of the bra class (segs[p - bra0]: the segment of bra pair p)
 };
 
 struct GradLaunch {
@@ -108,12 +110,7 @@ struct SchwarzLaunch {
   const double* pk;
   const RysArgs* ra;
   double* q2;
-  double* blk;  // staging of the (ab|ab) blocks of f-shell classes: npair x schwarz_block(c) doubles
 };
-
-// doubles of the Schwarz staging block per pair of pair class c (0 when the
-// class needs no staging); implemented with the class dispatch
-int schwarz_block(int pair_cls);
 
 void launch_jk(int bra_cls, int ket_cls, bool pure, const JKLaunch& a, hipStream_t s);
 void launch_schwarz(int pair_cls, bool pure, const SchwarzLaunch& a, hipStream_t s);
