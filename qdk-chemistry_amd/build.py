@@ -141,7 +141,7 @@ def gen_sources():
     os.makedirs(GEN, exist_ok=True)
     pcs = pair_classes(MAX_L)
     files = []
-    decls, jk_cases, sw_cases, gr_cases = [], [], [], []
+    decls, jk_cases, sw_cases, gr_cases, dn_cases = [], [], [], [], []
     head = ["// generated by build.py", '#include "../../eri_grad.hpp"', "namespace qfe {"]
     for b, (la, lb) in enumerate(pcs):
         for k, (lc, ld) in enumerate(pcs[: b + 1]):
@@ -186,6 +186,15 @@ def gen_sources():
             path = os.path.join(GEN, f"jkc_{tag}.hip")
             _write_if_changed(path, "\n".join(body + ["}  // namespace qfe"]) + "\n")
             files.append(path)
+            if not fcls:  # the class of the dense AO tensor (MO transforms, shells up to d)
+                dn = ["// generated by build.py", '#include "../../eri_dense_coop.hpp"', "namespace qfe {",
+                      f"void dense_cls_{tag}(const DenseLaunch& a, const RysArgs& ra, hipStream_t s) {{ "
+                      f"dense_coop<{la}, {lb}, {lc}, {ld}>(a, ra, s); }}", "}  // namespace qfe"]
+                decls.append(f"void dense_cls_{tag}(const DenseLaunch& a, const RysArgs& ra, hipStream_t s);")
+                dn_cases.append(f"  if (cb == {b} && ck == {k}) {{ dense_cls_{tag}(a, ra, s); return; }}")
+                path = os.path.join(GEN, f"dense_{tag}.hip")
+                _write_if_changed(path, "\n".join(dn) + "\n")
+                files.append(path)
             few = f" && a.coop && a.ntask <= {jk_coop_tasks(la, lb, lc, ld)}" if seg else ""
             jk_cases.append(f"  if (cb == {b} && ck == {k}{few}) {{ jkc_cls_{tag}(a, s); return; }}")
             if seg:
@@ -220,7 +229,8 @@ def gen_sources():
                 _write_if_changed(path, "\n".join(body) + "\n")
                 files.append(path)
             gr_cases.append(f"  if (cb == {b} && ck == {k}) {{ {' '.join(gcalls)} return; }}")
-    disp = ["// generated by build.py -- class dispatch", '#include "../../kernels.hpp"', "#include <stdexcept>",
+    disp = ["// generated by build.py -- class dispatch", '#include "../../kernels.hpp"',
+            '#include "../../eri_dense.hpp"', "#include <stdexcept>",
             "namespace qfe {"] + decls + [
         "void launch_jk(int cb, int ck, bool pure, const JKLaunch& a, hipStream_t s) {",
         '  if (!pure) throw std::runtime_error("cartesian bases are not compiled");'] + jk_cases + [
@@ -231,6 +241,8 @@ def gen_sources():
         "void launch_grad(int cb, int ck, bool pure, const GradLaunch& a, hipStream_t s) {",
         '  if (!pure) throw std::runtime_error("cartesian bases are not compiled");'] + gr_cases + [
         '  throw std::runtime_error("gradient class not compiled");', "}",
+        "void launch_dense(int cb, int ck, const DenseLaunch& a, const RysArgs& ra, hipStream_t s) {"] + dn_cases + [
+        '  throw std::runtime_error("dense class not compiled");', "}",
         f"int grad_max_l() {{ return {min(MAX_L, GRAD_MAX_L)}; }}", "}  // namespace qfe"]
     path = os.path.join(GEN, "dispatch.hip")
     _write_if_changed(path, "\n".join(disp) + "\n")
@@ -300,9 +312,12 @@ def _deps(src):
     name = os.path.basename(src)
     core = ["eri_core.hpp", "sph_coef.inc", "kernels.hpp"]
     if name == "dispatch.hip":
-        hs = ["kernels.hpp"]
+        hs = core + ["dfj.hpp", "eri_dense.hpp"]
     elif name.startswith("chunks"):
         hs = core + ["eri_class.hpp"]
+    elif name.startswith("dense_"):
+        hs = core + ["fixed_point.hpp", "eri_class.hpp", "eri_coop.hpp", "eri_jk_coop.hpp", "dfj.hpp", "eri_dense.hpp",
+                     "eri_dense_coop.hpp"]
     elif name.startswith("jkc_"):
         hs = core + ["fixed_point.hpp", "eri_class.hpp", "eri_coop.hpp", "eri_jk_coop.hpp"]
     elif name.startswith("gradc_"):

@@ -13,7 +13,6 @@
 
 #include <algorithm>
 #include <limits>
-#include <tuple>
 #include <utility>
 #include <cmath>
 #include <cstdio>
@@ -1742,8 +1741,8 @@ static void dense_tensor(const BasisHost& b, int dev, DevBuf<double>& T, size_t 
   std::vector<DevBuf<int>> ib;
   std::vector<DevBuf<double>> db;
   const DFBasisView v = DFJ::view(b, ib, db, 2, "MO transform: orbital");
-  // every unordered shell pair once, the higher l first, grouped by class
-  // and contraction length so that a wave's quartets mostly share them
+  // every unordered shell pair once, the higher l first, by class and
+  // contraction length
   std::vector<int2> pr;
   pr.reserve((size_t)b.nsh * (b.nsh + 1) / 2);
   for (int s1 = 0; s1 < b.nsh; ++s1)
@@ -1751,16 +1750,44 @@ static void dense_tensor(const BasisHost& b, int dev, DevBuf<double>& T, size_t 
       const bool swap = b.shells[s2].l > b.shells[s1].l;
       pr.push_back(int2{swap ? s2 : s1, swap ? s1 : s2});
     }
-  auto key = [&](const int2& p) {
-    const ShellHost &x = b.shells[p.x], &y = b.shells[p.y];
-    return std::make_tuple(x.l, y.l, x.a.size() * y.a.size());
+  auto cls = [&](const int2& p) {
+    const int l = b.shells[p.x].l;
+    return l * (l + 1) / 2 + b.shells[p.y].l;
   };
-  std::stable_sort(pr.begin(), pr.end(), [&](const int2& p, const int2& q) { return key(p) < key(q); });
+  auto len = [&](const int2& p) { return b.shells[p.x].a.size() * b.shells[p.y].a.size(); };
+  std::stable_sort(pr.begin(), pr.end(), [&](const int2& p, const int2& q) {
+    return std::make_pair(cls(p), len(p)) < std::make_pair(cls(q), len(q));
+  });
+  std::vector<int> prim0(pr.size());
+  std::vector<int> first(7, (int)pr.size());  // first pair of each class, s and p and d shells
+  size_t np = 0;
+  for (size_t i = 0; i < pr.size(); ++i) {
+    prim0[i] = (int)np;
+    np += len(pr[i]);
+    for (int c = cls(pr[i]); c >= 0 && first[c] == (int)pr.size(); --c) first[c] = (int)i;
+  }
+  if (np > (size_t)std::numeric_limits<int>::max()) throw Unsupported("MO transform: too many primitive pairs");
   DevBuf<int2> pairs;
+  DevBuf<int> off;
+  DevBuf<PairHdr> hdr;
+  DevBuf<double4> ppos;
+  DevBuf<double> pk;
   pairs.upload(pr, nullptr);
+  off.upload(prim0, nullptr);
+  hdr.alloc(pr.size());
+  ppos.alloc(np);
+  pk.alloc(np);
   T.alloc(n4);
-  launch_eri_dense(v, tb.ra, tb.sph, pairs.p, T.p, nullptr);
+  launch_dense_pairs(v, pairs.p, off.p, (int)pr.size(), hdr.p, ppos.p, pk.p, nullptr);
   HIP_CHECK(hipGetLastError());
+  for (int cb = 5; cb >= 0; --cb)
+    for (int ck = cb; ck >= 0; --ck) {
+      const DenseLaunch a{hdr.p + first[cb], first[cb + 1] - first[cb], hdr.p + first[ck], first[ck + 1] - first[ck],
+                          cb == ck, ppos.p, pk.p, b.nbf, T.p};
+      if (a.nbra <= 0 || a.nket <= 0) continue;
+      launch_dense(cb, ck, a, tb.ra, nullptr);
+      HIP_CHECK(hipGetLastError());
+    }
   HIP_CHECK(hipDeviceSynchronize());
 }
 
