@@ -1322,7 +1322,7 @@ static const OneBodyTables& one_body_tables(int device) {
 
 // flat copy of a basis on the current device, for one call
 struct OneBodyDevice {
-  DevBuf<int> l, atom, po, bf0;
+  DevBuf<int> l, atom, po, bf0, by_l;
   DevBuf<double> cen, exps, coefs, Z, R;
   OneBodyView view{};
   OneBodyDevice(const BasisHost& b, const double* sph) {
@@ -1339,7 +1339,11 @@ struct OneBodyDevice {
       hk.insert(hk.end(), sh.c.begin(), sh.c.end());
       hpo[s + 1] = (int)he.size();
     }
+    std::vector<int> hby(b.nsh);
+    std::iota(hby.begin(), hby.end(), 0);
+    std::stable_sort(hby.begin(), hby.end(), [&](int x, int y) { return hl[x] < hl[y]; });
     l.upload(hl, nullptr);
+    by_l.upload(hby, nullptr);
     atom.upload(hat, nullptr);
     po.upload(hpo, nullptr);
     bf0.upload(hbf, nullptr);
@@ -1348,8 +1352,10 @@ struct OneBodyDevice {
     coefs.upload(hk, nullptr);
     Z.upload(b.Z, nullptr);
     R.upload(b.R, nullptr);
-    view = OneBodyView{l.p, atom.p, po.p, bf0.p, cen.p, exps.p, coefs.p, Z.p, R.p, sph, b.nsh, b.natoms, b.nbf,
-                       b.pure ? 1 : 0};
+    view = OneBodyView{l.p, atom.p, po.p, bf0.p, cen.p, exps.p, coefs.p, Z.p, R.p, sph, by_l.p, {0, 0, 0, 0, 0},
+                       b.nsh, b.natoms, b.nbf, b.pure ? 1 : 0};
+    for (int x : hl)
+      for (int k = x + 1; k < 5; ++k) ++view.nl[k];
   }
 };
 
@@ -1649,10 +1655,12 @@ int qfe_one_body_grad_gpu(const qfe_basis* basis, int op, const double* W, doubl
     const size_t nn = (size_t)b.nbf * b.nbf;
     qfe::DevBuf<double> w, g;
     w.alloc(nn);
-    g.alloc(3 * (size_t)b.natoms);
+    g.alloc(qfe::kGradCopies * 3 * (size_t)b.natoms);
     HIP_CHECK(hipMemcpy(w.p, W, sizeof(double) * nn, hipMemcpyHostToDevice));
-    HIP_CHECK(hipMemset(g.p, 0, sizeof(double) * 3 * (size_t)b.natoms));
-    qfe::launch_one_body_grad(d.view, tb.ra, op, w.p, g.p, nullptr);
+    HIP_CHECK(hipMemset(g.p, 0, sizeof(double) * qfe::kGradCopies * 3 * (size_t)b.natoms));
+    qfe::launch_one_body_grad(d.view, tb.ra, op, w.p, g.p, qfe::kGradCopies, nullptr);
+    HIP_CHECK(hipGetLastError());
+    qfe::launch_fold_copies(g.p, 3 * b.natoms, qfe::kGradCopies, nullptr);
     HIP_CHECK(hipGetLastError());
     HIP_CHECK(hipMemcpy(grad, g.p, sizeof(double) * 3 * (size_t)b.natoms, hipMemcpyDeviceToHost));
   });

@@ -11,7 +11,8 @@ namespace qfe {
 // range [po[s], po[s+1]) into exps/coefs (normalised contraction
 // coefficients), first output function bf0[s]; per atom the nuclear charge
 // seen by the electrons Z and the position R (3 doubles); the solid-harmonic
-// table sph[l][m][c] (5 x 9 x 15 doubles).  Shells up to l = 3.
+// table sph[l][m][c] (5 x 9 x 15 doubles).  Shells up to l = 3; by_l holds the
+// shell indices by angular momentum, those of l in [nl[l], nl[l + 1]).
 struct OneBodyView {
   const int* l;
   const int* atom;
@@ -23,13 +24,16 @@ struct OneBodyView {
   const double* Z;
   const double* R;
   const double* sph;
+  const int* by_l;
+  int nl[5];
   int nsh, natoms, nbf, pure;
 };
 
 // op 0 = S, 1 = T, 2 = V into out (nbf x nbf, row-major, device)
 void launch_one_body(const OneBodyView& b, const RysArgs& ra, int op, double* out, hipStream_t s);
-// grad[natoms][3] (device, zeroed by the caller) += sum_mn W_mn dO_mn/dR
-void launch_one_body_grad(const OneBodyView& b, const RysArgs& ra, int op, const double* W, double* grad,
+// sum_mn W_mn dO_mn/dR added to ncopy copies of grad[natoms][3] (device, 3
+// natoms apart, zeroed by the caller, a power of two of them)
+void launch_one_body_grad(const OneBodyView& b, const RysArgs& ra, int op, const double* W, double* grad, int ncopy,
                           hipStream_t s);
 
 }  // namespace qfe
