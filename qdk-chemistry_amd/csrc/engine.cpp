@@ -322,7 +322,7 @@ struct Engine {
   double* jbuf_p = nullptr;
   unsigned long long* jmask_p = nullptr;
   DevBuf<int> sh_bf0_d, sh_nf_d;
-  DevBuf<int4> kets_d;        // per pair {prim0, nprim, sa, sb} (class kernels' ket side)
+  DevBuf<int4> kets_d;        // per pair {prim0, nprim, pstride, sa | sb << 16} (class kernels' ket side)
   DevBuf<double4> shells_d;   // per shell {x, y, z, first AO}
   DevBuf<double> Pn_d, pmax_d;  // shell-block density norms (nsh x nsh) and their maximum
   DevBuf<int> bad_d;
@@ -506,7 +506,7 @@ struct Engine {
           pa.push_back(a);
         }
       h.nprim = (int)ppos.size() - h.prim0;
-      h.pad = 0;
+      h.pstride = 1;
     }
     prim_pairs = (long long)ppos.size();
     const int npair = (int)hdr.size();
@@ -547,40 +547,48 @@ struct Engine {
     });
     pairs_h.resize(npair);
     Q_h.resize(npair);
-    std::vector<double4> ppos2;
-    std::vector<double> pk2, pa2;
-    ppos2.reserve(ppos.size());
-    pk2.reserve(pk.size());
-    for (int i = 0; i < npair; ++i) {
-      PairHdr h = hdr[ord[i]];
-      const int old0 = h.prim0;
-      h.prim0 = (int)ppos2.size();
-      // primitives by screening factor, largest first: the primitive
-      // quartets a build keeps form a prefix of each pair's list
-      std::vector<int> po(h.nprim);
-      std::iota(po.begin(), po.end(), 0);
-      std::stable_sort(po.begin(), po.end(), [&](int x, int y) {
-        return prim_sig(ppos[old0 + x].x, pk[old0 + x]) > prim_sig(ppos[old0 + y].x, pk[old0 + y]);
-      });
-      for (int k : po) {
-        ppos2.push_back(ppos[old0 + k]);
-        pk2.push_back(pk[old0 + k]);
-        pa2.push_back(pa[old0 + k]);
-      }
-      pairs_h[i] = h;
-      Q_h[i] = Q[ord[i]];
-    }
     // buckets
     buckets_h.clear();
     bucket_cls_h.clear();
     pair_bucket_h.assign(npair, 0);
     for (int i = 0; i < npair;) {
       int j = i;
-      while (j < npair && pairs_h[j].cls == pairs_h[i].cls && pairs_h[j].nprim == pairs_h[i].nprim) ++j;
+      while (j < npair && hdr[ord[j]].cls == hdr[ord[i]].cls && hdr[ord[j]].nprim == hdr[ord[i]].nprim) ++j;
       for (int k = i; k < j; ++k) pair_bucket_h[k] = (int)buckets_h.size();
       buckets_h.push_back(make_int2(i, j));
-      bucket_cls_h.push_back(pairs_h[i].cls);
+      bucket_cls_h.push_back(hdr[ord[i]].cls);
       i = j;
+    }
+    // Primitive tables, transposed inside a bucket: entry k of its pair i at
+    // first + k (pairs of the bucket) + i, so that lanes on neighbouring ket
+    // pairs read neighbouring entries.  Each pair's primitives go by screening
+    // factor, largest first: the primitive quartets a build keeps form a
+    // prefix of each pair's list.
+    std::vector<double4> ppos2(ppos.size());
+    std::vector<double> pk2(pk.size()), pa2(pa.size());
+    size_t first = 0;
+    for (const int2& bk : buckets_h) {
+      const int size = bk.y - bk.x;
+      for (int i = bk.x; i < bk.y; ++i) {
+        PairHdr h = hdr[ord[i]];
+        const int old0 = h.prim0;
+        h.prim0 = (int)first + (i - bk.x);
+        h.pstride = size;
+        std::vector<int> po(h.nprim);
+        std::iota(po.begin(), po.end(), 0);
+        std::stable_sort(po.begin(), po.end(), [&](int x, int y) {
+          return prim_sig(ppos[old0 + x].x, pk[old0 + x]) > prim_sig(ppos[old0 + y].x, pk[old0 + y]);
+        });
+        for (int k = 0; k < h.nprim; ++k) {
+          const size_t e = (size_t)h.prim0 + (size_t)k * size;
+          ppos2[e] = ppos[old0 + po[k]];
+          pk2[e] = pk[old0 + po[k]];
+          pa2[e] = pa[old0 + po[k]];
+        }
+        pairs_h[i] = h;
+        Q_h[i] = Q[ord[i]];
+      }
+      first += (size_t)size * (size_t)hdr[ord[bk.x]].nprim;
     }
     // work items ordered by class pair, then (bra bucket, ket bucket, bra pair)
     const int nb = (int)buckets_h.size();
@@ -635,7 +643,8 @@ struct Engine {
     {
       std::vector<int4> kr(npair);
       for (int i = 0; i < npair; ++i)
-        kr[i] = make_int4(pairs_h[i].prim0, pairs_h[i].nprim, pairs_h[i].sa, pairs_h[i].sb);
+        kr[i] = make_int4(pairs_h[i].prim0, pairs_h[i].nprim, pairs_h[i].pstride,
+                          (int)((unsigned)pairs_h[i].sa | (unsigned)pairs_h[i].sb << 16));
       kets_d.upload(kr, stream);
       std::vector<double4> sr(nsh);
       for (int s2 = 0; s2 < nsh; ++s2)

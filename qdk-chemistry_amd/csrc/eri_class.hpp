@@ -127,12 +127,14 @@ struct SegRows {
   static constexpr int NR = NMA + NMB;  // LDS rows: a functions, then b functions
 };
 
-// The ket pair of a task from its 16-byte record {prim0, nprim, sa, sb} and
+// The ket pair of a task from its 16-byte record {prim0, nprim, pstride,
+// sa | sb << 16} and
 // the shell table {x, y, z, first AO} (nsh entries, small enough to stay in
 // L2): 16 bytes per task from the pair table instead of the 80-byte header
 QFE_DI PairHdr ket_record(const int4* __restrict__ kets, const double4* __restrict__ shells, int p) {
   const int4 r = kets[p];
-  const double4 c = shells[r.z], d = shells[r.w];
+  const int sa = r.w & 0xffff, sb = (int)((unsigned)r.w >> 16);
+  const double4 c = shells[sa], d = shells[sb];
   PairHdr h;
   h.A[0] = c.x;
   h.A[1] = c.y;
@@ -142,12 +144,12 @@ QFE_DI PairHdr ket_record(const int4* __restrict__ kets, const double4* __restri
   h.B[2] = d.z;
   h.prim0 = r.x;
   h.nprim = r.y;
-  h.sa = r.z;
-  h.sb = r.w;
+  h.sa = sa;
+  h.sb = sb;
   h.bfa = (int)c.w;
   h.bfb = (int)d.w;
   h.cls = 0;
-  h.pad = 0;
+  h.pstride = r.z;
   return h;
 }
 

@@ -68,10 +68,10 @@ QFE_HD constexpr double sph_coef(int l, bool pure, int m, int c) {
 struct PairHdr {        // one significant shell pair (80 B)
   double A[3];          // centre of shell a
   double B[3];          // centre of shell b
-  int prim0, nprim;     // range in the primitive-pair arrays
+  int prim0, nprim;     // primitive pair k is entry prim0 + k pstride of their arrays
   int sa, sb;           // shell indices (AO order of the reference)
   int bfa, bfb;         // first AO of each shell
-  int cls, pad;
+  int cls, pstride;
 };
 
 // primitive pair: ppos = (p, Px, Py, Pz); pk = c_a c_b exp(-ab/p |AB|^2) / p
@@ -411,7 +411,9 @@ QFE_DI void contract_chunk(const PairHdr& bra, const PairHdr& ket,
   // following each other across the test (a primitive past the cut still
   // lies in its pair's range: the reads stay in bounds)
   using V4 = typename Vec4<R>::type;
-  for (int ik = ket.prim0; ik < ket.prim0 + ket.nprim; ++ik) {
+  const int kend = ket.prim0 + ket.nprim * ket.pstride;
+  const int bend = bra.prim0 + bra.nprim * bra.pstride;
+  for (int ik = ket.prim0; ik < kend; ik += ket.pstride) {
     const R sk = sig[ik];
     V4 Q;
     R Kk, h2q;  // h2q: used from a ket (pp) or (ds) on
@@ -425,7 +427,7 @@ QFE_DI void contract_chunk(const PairHdr& bra, const PairHdr& ket,
     const R blim = lnp - sk;
     const R q = Q.x;
     const R QCx = Q.y - Cx, QCy = Q.z - Cy, QCz = Q.w - Cz;
-    for (int ib0 = bra.prim0; ib0 < bra.prim0 + bra.nprim; ++ib0) {
+    for (int ib0 = bra.prim0; ib0 < bend; ib0 += bra.pstride) {
       int ib = ib0;
       bool on = true;
       V4 P;

@@ -48,7 +48,7 @@ __global__ __launch_bounds__(256) void k_dense_pairs(DFBasisView b, const int2* 
     h.bfa = b.bf0[sa];
     h.bfb = b.bf0[sb];
     h.cls = b.l[sa] * (b.l[sa] + 1) / 2 + b.l[sb];
-    h.pad = 0;
+    h.pstride = 1;
     hdr[i] = h;
   }
 }

@@ -129,14 +129,16 @@ QFE_DI void grad_task(int2 tk, const PairHdr* __restrict__ pairs, const double4*
   constexpr double TWO_PI_52 = 34.98683665524972;
   const double ABx = bra.A[0] - bra.B[0], ABy = bra.A[1] - bra.B[1], ABz = bra.A[2] - bra.B[2];
   const double CDx = ket.A[0] - ket.B[0], CDy = ket.A[1] - ket.B[1], CDz = ket.A[2] - ket.B[2];
-  for (int ik = ket.prim0; ik < ket.prim0 + ket.nprim; ++ik) {
+  const int kend = ket.prim0 + ket.nprim * ket.pstride;
+  const int bend = bra.prim0 + bra.nprim * bra.pstride;
+  for (int ik = ket.prim0; ik < kend; ik += ket.pstride) {
     const double4 Q = ppos[ik];
     const double Kk = pk[ik];
     const double q = Q.x;
     const double tg = 2.0 * pa[ik];  // 2 gamma (exponent on centre C)
     const double QCx = Q.y - ket.A[0], QCy = Q.z - ket.A[1], QCz = Q.w - ket.A[2];
     const double h2q = 0.5 * frcp(q);
-    for (int ib = bra.prim0; ib < bra.prim0 + bra.nprim; ++ib) {
+    for (int ib = bra.prim0; ib < bend; ib += bra.pstride) {
       const double4 Pp = ppos[ib];
       const double Kb = pk[ib];
       const double p = Pp.x;

@@ -99,7 +99,7 @@ __global__ __launch_bounds__(G::BLK) void k_eri_grad_coop(
       if (tid < 3 * nc) {
         const int i = tid / 3, x = tid % 3;
         const int pr = (g0 + i) / G::NR, r = (g0 + i) % G::NR;
-        const int ib = bra.prim0 + pr % bra.nprim, ik = ket.prim0 + pr / bra.nprim;
+        const int ib = bra.prim0 + pr % bra.nprim * bra.pstride, ik = ket.prim0 + pr / bra.nprim * ket.pstride;
         const double4 Pp = ppos[ib], Q = ppos[ik];
         const double p = Pp.x, q = Q.x;
         const double PQx = Pp.y - Q.y, PQy = Pp.z - Q.z, PQz = Pp.w - Q.w;

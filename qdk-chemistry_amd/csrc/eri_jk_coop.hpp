@@ -77,10 +77,15 @@ QFE_DI void coop_transform(const double* in, double* out, int tid) {
   }
 }
 
-// table offsets of a thread's (a, b, c) triples, and its slice of a batch
+// table offsets of a thread's (a, b, c) triples (10 bits each: a table holds at
+// most 257 entries), and its slice of a batch
 template <class G>
 struct CoopOffsets {
-  int ox[G::NIT], oy[G::NIT], oz[G::NIT], sl;
+  static_assert(3 * G::NI < 1024, "packed offsets");
+  int o[G::NIT], sl;
+  QFE_DI int x(int it) const { return o[it] & 1023; }
+  QFE_DI int y(int it) const { return o[it] >> 10 & 1023; }
+  QFE_DI int z(int it) const { return o[it] >> 20; }
   QFE_DI explicit CoopOffsets(int tid) {
     sfor<G::NIT>([&](auto it) {
       const int k = (tid + it * G::BLK) % G::NABC;
@@ -88,9 +93,8 @@ struct CoopOffsets {
       coop_xyz<G::LA>(k / (G::NB * G::NC), ax, ay, az);
       coop_xyz<G::LB>(k / G::NC % G::NB, bx, by, bz);
       coop_xyz<G::LC>(k % G::NC, cx, cy, cz);
-      ox[it] = ax * G::SA + bx * G::SB + cx * G::SC;
-      oy[it] = G::NI + ay * G::SA + by * G::SB + cy * G::SC;
-      oz[it] = 2 * G::NI + az * G::SA + bz * G::SB + cz * G::SC;
+      o[it] = (ax * G::SA + bx * G::SB + cx * G::SC) | (G::NI + ay * G::SA + by * G::SB + cy * G::SC) << 10 |
+              (2 * G::NI + az * G::SA + bz * G::SB + cz * G::SC) << 20;
     });
     sl = G::NSL > 1 ? tid / G::NABC : 0;
   }
@@ -114,9 +118,9 @@ __device__ __forceinline__ double* coop_quartet(const PairHdr& bra, const PairHd
     const double sb0 = sig[bra.prim0], sk0 = sig[ket.prim0];
     nbp = nkp = 0;
     for (int i = lane; i - lane < bra.nprim; i += 64)
-      nbp += __popcll(__ballot(i < bra.nprim && !(sig[bra.prim0 + (i < bra.nprim ? i : 0)] + sk0 < lnp)));
+      nbp += __popcll(__ballot(i < bra.nprim && !(sig[bra.prim0 + (i < bra.nprim ? i : 0) * bra.pstride] + sk0 < lnp)));
     for (int i = lane; i - lane < ket.nprim; i += 64)
-      nkp += __popcll(__ballot(i < ket.nprim && !(sig[ket.prim0 + (i < ket.nprim ? i : 0)] + sb0 < lnp)));
+      nkp += __popcll(__ballot(i < ket.nprim && !(sig[ket.prim0 + (i < ket.nprim ? i : 0) * ket.pstride] + sb0 < lnp)));
   }
   double acc[G::NIT][G::ND];
   sfor<G::NIT>([&](auto it) { sfor<G::ND>([&](auto d) { acc[it][d] = 0.0; }); });
@@ -126,7 +130,7 @@ __device__ __forceinline__ double* coop_quartet(const PairHdr& bra, const PairHd
     if (tid < 3 * nc) {
       const int i = tid / 3, x = tid % 3;
       const int pr = (g0 + i) / G::NR, r = (g0 + i) % G::NR;
-      const int ib = bra.prim0 + pr % nbp, ik = ket.prim0 + pr / nbp;
+      const int ib = bra.prim0 + pr % nbp * bra.pstride, ik = ket.prim0 + pr / nbp * ket.pstride;
       const double4 Pp = ppos[ib], Q = ppos[ik];
       const double p = Pp.x, q = Q.x;
       const double PQx = Pp.y - Q.y, PQy = Pp.z - Q.z, PQz = Pp.w - Q.w;
@@ -153,9 +157,9 @@ __device__ __forceinline__ double* coop_quartet(const PairHdr& bra, const PairHd
       sfor<G::NIT>([&](auto it) {
         double vx[G::LD + 1], vy[G::LD + 1], vz[G::LD + 1];
         sfor<G::LD + 1>([&](auto d) {
-          vx[d] = tb[of.ox[it] + d];
-          vy[d] = tb[of.oy[it] + d];
-          vz[d] = tb[of.oz[it] + d];
+          vx[d] = tb[of.x(it) + d];
+          vy[d] = tb[of.y(it) + d];
+          vz[d] = tb[of.z(it) + d];
         });
         sfor<G::ND>([&](auto d) {
           constexpr int dx = cart_x(G::LD, d), dy = cart_y(G::LD, d), dz = cart_z(G::LD, d);

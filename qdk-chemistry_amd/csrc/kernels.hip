@@ -579,11 +579,11 @@ __global__ __launch_bounds__(256) void k_count_prims(const int2* __restrict__ ta
     const PairHdr bra = pairs[tk.x], ket = pairs[tk.y];
     const R lnp = prim_ln_cut<R>(pmax, prim_screen);
     const R sb0 = sig[bra.prim0];
-    for (int ik = ket.prim0; ik < ket.prim0 + ket.nprim; ++ik) {
+    for (int ik = ket.prim0; ik < ket.prim0 + ket.nprim * ket.pstride; ik += ket.pstride) {
       const R sk = sig[ik];
       if (sk + sb0 < lnp) break;
       const R blim = lnp - sk;
-      for (int ib = bra.prim0; ib < bra.prim0 + bra.nprim; ++ib) {
+      for (int ib = bra.prim0; ib < bra.prim0 + bra.nprim * bra.pstride; ib += bra.pstride) {
         if (sig[ib] < blim) break;
         ++n;
       }
