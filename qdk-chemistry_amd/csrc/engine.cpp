@@ -1028,12 +1028,12 @@ struct Engine {
     // the classes are independent (their contributions are added with
     // atomics): spread over the streams by work like those of a J/K build
     const int nst = 1 + (int)side.size();
-    std::vector<std::pair<double, int>> jobs;  // (quartets x functions per quartet, class pair)
+    std::vector<std::pair<double, int>> jobs;  // (work, class pair)
     for (int cp = 0; cp < ncp; ++cp) {
       const long long n = bval[cp + 1] - bval[cp];
       if (n <= 0) continue;
       nq += n;
-      jobs.push_back({(double)n * nfun_pair_class(cp_bra[cp]) * nfun_pair_class(cp_ket[cp]), cp});
+      jobs.push_back({class_cost(0, cp), cp});
     }
     if (nst > 1) {
       std::stable_sort(jobs.begin(), jobs.end(), [](const auto& x, const auto& y) { return x.first > y.first; });
@@ -1076,6 +1076,18 @@ struct Engine {
     stats.ms_total = t01 + t12;
   }
 
+  // Estimated work of a class of the last screen(), to deal the classes over
+  // the streams: about 2 + nf units a primitive quartet (nf functions a
+  // quartet; (ss|ss) 2.7, (ps|ps) 11, (pp|ps) 25, (dp|pp) 500 ps each) and 3 nf
+  // for a quartet's digestion.  With the functions of the quartets alone,
+  // (ss|ss) came last, whose contracted quartets are the longest chains.
+  double class_cost(int prec, int cp) const {
+    const size_t ncp = cp_bra.size();
+    const double* c = cstat_h.data() + 2 * (size_t)prec * ncp;  // quartets, then primitive quartets
+    const double nf = (double)nfun_pair_class(cp_bra[cp]) * nfun_pair_class(cp_ket[cp]);
+    return c[ncp + cp] * (2.0 + nf) + 3.0 * c[cp] * nf;
+  }
+
   // Class kernels and J_cd reduction of density dP over the task list of the
   // last screen(): J += Coulomb (dJ null: skipped), K += exchange scaled by
   // kscale (dK null: skipped).  J and K must be zeroed by the caller.
@@ -1091,8 +1103,8 @@ struct Engine {
     double* Jd = det ? nullptr : dJ;
     nq = nq32 = 0;
     // the class kernels over 1 + side.size() streams: the classes by work
-    // (quartets x functions per quartet), largest first, each to the stream
-    // with the least work so far; profiled engines keep one stream
+    // (class_cost), largest first, each to the stream with the least work so
+    // far; profiled engines keep one stream
     const int nst = profile ? 1 : 1 + (int)side.size();
     struct Job {
       double cost;
@@ -1105,7 +1117,7 @@ struct Engine {
         const long long n = b[cp + 1] - b[cp];
         if (n <= 0) continue;
         (prec ? nq32 : nq) += n;
-        jobs.push_back({(double)n * nfun_pair_class(cp_bra[cp]) * nfun_pair_class(cp_ket[cp]), prec, cp});
+        jobs.push_back({class_cost(prec, cp), prec, cp});
       }
     }
     if (nst > 1)
