@@ -4,8 +4,9 @@
 // full square of the reference's INCORE DF engine,
 // scf/src/eri/INCORE/incore_impl_df.cpp:53-80), and the two-centre metric
 // V[P][Q] = (P|Q), kept in HBM.  The
-// build itself (X = B . vec(D), V c = X, J = B^T c; incore_impl_df.cpp:
-// 81-200) runs in engine.cpp with rocBLAS and rocSOLVER.
+// build itself is X = B . vec(D), V c = X, J = B^T c (incore_impl_df.cpp:
+// 81-200); the last product, a plain GEMV that rocBLAS streams at 5.7 TB/s,
+// runs in engine.cpp.
 //
 // The integrals are Rys quadrature with runtime angular momenta (orbital
 // shells up to d, auxiliary shells up to g): per primitive triple and root,
@@ -279,9 +280,238 @@ __global__ __launch_bounds__(256) void k_df_unpack(const double* __restrict__ j,
   J[e] = j[hi * (hi + 1) / 2 + lo];
 }
 
+// x = B d reads B once and is bound by HBM.  A block takes kDfRows rows x
+// kDfChunk elements, so that d is read from L2 once for kDfRows rows: 0.87 ms
+// (6.1 TB/s) at (H2O)32/def2-SVP, where rocBLAS's transposed GEMV took 1.55 ms.
+// Rows start at any multiple of 8 bytes (np may be odd), so the loads are
+// single doubles.
+constexpr int kDfRows = 16;
+__global__ __launch_bounds__(256) void k_df_dots(const double* __restrict__ B, const double* __restrict__ d,
+                                                 size_t np, int naux, int nchunk, double* __restrict__ part) {
+  constexpr int N = kDfChunk / 256;
+  __shared__ double sm[4][kDfRows];
+  const int tid = (int)threadIdx.x, lane = tid & 63;
+  const size_t c0 = (size_t)blockIdx.x * kDfChunk + tid;
+  const int r0 = (int)blockIdx.y * kDfRows, nr = naux - r0 < kDfRows ? naux - r0 : kDfRows;
+  double dv[N];
+#pragma unroll
+  for (int k = 0; k < N; ++k) dv[k] = c0 + 256 * k < np ? d[c0 + 256 * k] : 0.0;
+  for (int r = 0; r < nr; ++r) {
+    const double* row = B + (size_t)(r0 + r) * np;
+    double bv[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) bv[k] = c0 + 256 * k < np ? row[c0 + 256 * k] : 0.0;
+    double s = 0.0;
+#pragma unroll
+    for (int k = 0; k < N; ++k) s = fma(bv[k], dv[k], s);
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    if (lane == 0) sm[tid >> 6][r] = s;
+  }
+  __syncthreads();
+  if (tid < nr) part[(size_t)(r0 + tid) * nchunk + blockIdx.x] = sm[0][tid] + sm[1][tid] + sm[2][tid] + sm[3][tid];
+}
+
+// x[P] = sum of its chunks, one wave per P
+__global__ __launch_bounds__(256) void k_df_sum(const double* __restrict__ part, int naux, int nchunk,
+                                                double* __restrict__ x) {
+  const int p = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6), lane = (int)(threadIdx.x & 63);
+  if (p >= naux) return;
+  double s = 0.0;
+  for (int k = lane; k < nchunk; k += 64) s += part[(size_t)p * nchunk + k];
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+  if (lane == 0) x[p] = s;
+}
+
+// Triangular solves by blocks of kDfBlock rows: rocSOLVER's potrs spent 0.86 ms
+// in two substitutions of 2272 rows, one dependent step after another.  Here a
+// launch per block solves its unknowns with the inverse of the diagonal block
+// and applies them to all the rows that remain.  The product with the inverse
+// alone would be a digit short of substitution (residual 2e-15 of |b| instead
+// of 1.4e-16 at a metric of condition 6e10), so it is corrected once by the
+// block's own residual, which brings it to 1.3e-16.  36 launches of 10-12 us:
+// 0.41 ms.
+__global__ __launch_bounds__(kDfBlock) void k_df_inverses(const double* __restrict__ L, int n,
+                                                          double* __restrict__ dinv) {
+  // thread j: column j of the inverse of block blockIdx.x, by substitution
+  const int b0 = (int)blockIdx.x * kDfBlock, nb = n - b0 < kDfBlock ? n - b0 : kDfBlock, j = (int)threadIdx.x;
+  double* D = dinv + (size_t)b0 * kDfBlock;
+  if (j >= nb) {
+    for (int i = 0; i < nb; ++i) D[(size_t)i * kDfBlock + j] = 0.0;
+    return;
+  }
+  for (int i = 0; i < j; ++i) D[(size_t)i * kDfBlock + j] = 0.0;
+  for (int i = j; i < nb; ++i) {
+    double s = i == j ? 1.0 : 0.0;
+    for (int m = j; m < i; ++m) s = fma(-L[(size_t)(b0 + m) * n + b0 + i], D[(size_t)m * kDfBlock + j], s);
+    D[(size_t)i * kDfBlock + j] = s / L[(size_t)(b0 + i) * n + b0 + i];
+  }
+}
+
+// What a step reads does not depend on the unknowns before it, so every load is
+// issued before the first product: a step costs one memory latency.
+constexpr int kDfThreads = 4 * kDfBlock, kDfPer = kDfBlock / 4;
+
+// zb = the unknowns of block b0 for the right-hand side r: with the block
+// itself (FWD) or its transpose.  rows: sixteen lanes a row, along contiguous
+// k, four rows a lane; cols: one lane a row and quarter of k, partial sums
+// through LDS.
+template <bool FWD>
+__device__ __forceinline__ void df_block(const double* __restrict__ L, const double* __restrict__ dinv, int n, int b0,
+                                         int nb, const double* __restrict__ r, double* rb, double* zb, double* res,
+                                         double (*part)[kDfBlock]) {
+  constexpr int NK = kDfBlock / 16, RS = kDfThreads / 16, NR = kDfBlock / RS;
+  const int tid = (int)threadIdx.x, i = tid >> 4, h = tid & 15, c = tid & (kDfBlock - 1), q = tid / kDfBlock;
+  double rows[NR][NK], cols[kDfPer];
+#pragma unroll
+  for (int p = 0; p < NR; ++p)
+#pragma unroll
+    for (int m = 0; m < NK; ++m) {
+      const int k = h + 16 * m, row = i + RS * p;
+      if constexpr (FWD)
+        rows[p][m] = k <= row && row < nb ? dinv[(size_t)(b0 + row) * kDfBlock + k] : 0.0;
+      else
+        rows[p][m] = k >= row && k < nb ? L[(size_t)(b0 + row) * n + b0 + k] : 0.0;
+    }
+#pragma unroll
+  for (int m = 0; m < kDfPer; ++m) {
+    const int k = q * kDfPer + m;
+    if constexpr (FWD)
+      cols[m] = k <= c && c < nb ? L[(size_t)(b0 + k) * n + b0 + c] : 0.0;
+    else
+      cols[m] = k >= c && k < nb ? dinv[(size_t)(b0 + k) * kDfBlock + c] : 0.0;
+  }
+  if (tid < kDfBlock) rb[tid] = tid < nb ? r[b0 + tid] : 0.0;
+  __syncthreads();
+  auto by_rows = [&](const double* v, double* out) {  // valid in the first lane of a row
+#pragma unroll
+    for (int p = 0; p < NR; ++p) out[p] = 0.0;
+#pragma unroll
+    for (int m = 0; m < NK; ++m) {
+      const double vk = v[h + 16 * m];
+#pragma unroll
+      for (int p = 0; p < NR; ++p) out[p] = fma(rows[p][m], vk, out[p]);
+    }
+#pragma unroll
+    for (int p = 0; p < NR; ++p)
+      for (int o = 8; o > 0; o >>= 1) out[p] += __shfl_xor(out[p], o);
+  };
+  auto by_cols = [&](const double* v) {  // valid in the first kDfBlock threads
+    double s = 0.0;
+#pragma unroll
+    for (int m = 0; m < kDfPer; ++m) s = fma(cols[m], v[q * kDfPer + m], s);
+    part[q][c] = s;
+    __syncthreads();
+    return (part[0][c] + part[1][c]) + (part[2][c] + part[3][c]);
+  };
+  if constexpr (FWD) {
+    double z[NR], dz[NR];
+    by_rows(rb, z);
+#pragma unroll
+    for (int p = 0; p < NR; ++p)
+      if (h == 0) zb[i + RS * p] = z[p];
+    __syncthreads();
+    const double t = by_cols(zb);
+    if (q == 0) res[c] = rb[c] - t;
+    __syncthreads();
+    by_rows(res, dz);
+#pragma unroll
+    for (int p = 0; p < NR; ++p)
+      if (h == 0) zb[i + RS * p] = z[p] + dz[p];
+  } else {
+    const double z = by_cols(rb);
+    if (q == 0) zb[c] = z;
+    __syncthreads();
+    double t[NR];
+    by_rows(zb, t);
+#pragma unroll
+    for (int p = 0; p < NR; ++p)
+      if (h == 0) res[i + RS * p] = rb[i + RS * p] - t[p];
+    __syncthreads();
+    const double dz = by_cols(res);
+    if (q == 0) zb[c] = z + dz;
+  }
+  __syncthreads();
+}
+
+// forward step: y of block b0 (every thread block forms it, the first stores
+// it), then x -= L y for the rows below, kDfBlock rows a thread block
+__global__ __launch_bounds__(kDfThreads) void k_df_forward(const double* __restrict__ L,
+                                                           const double* __restrict__ dinv, int n, int b0,
+                                                           double* __restrict__ x, double* __restrict__ y) {
+  __shared__ double rb[kDfBlock], zb[kDfBlock], res[kDfBlock], part[4][kDfBlock];
+  const int tid = (int)threadIdx.x, c = tid & (kDfBlock - 1), q = tid / kDfBlock;
+  const int nb = n - b0 < kDfBlock ? n - b0 : kDfBlock, i = b0 + nb + (int)blockIdx.x * kDfBlock + c;
+  double u[kDfPer];
+#pragma unroll
+  for (int m = 0; m < kDfPer; ++m) {
+    const int k = q * kDfPer + m;
+    u[m] = i < n && k < nb ? L[(size_t)(b0 + k) * n + i] : 0.0;
+  }
+  df_block<true>(L, dinv, n, b0, nb, x, rb, zb, res, part);
+  if (blockIdx.x == 0 && tid < nb) y[b0 + tid] = zb[tid];
+  double s = 0.0;
+#pragma unroll
+  for (int m = 0; m < kDfPer; ++m) s = fma(u[m], zb[q * kDfPer + m], s);
+  part[q][c] = s;
+  __syncthreads();
+  if (q == 0 && i < n) x[i] -= (part[0][c] + part[1][c]) + (part[2][c] + part[3][c]);
+}
+
+// backward step: x of block b0 from y, then y -= L^T x for the rows above, one
+// row a wave at a time (a column of L is contiguous)
+__global__ __launch_bounds__(kDfThreads) void k_df_backward(const double* __restrict__ L,
+                                                            const double* __restrict__ dinv, int n, int b0,
+                                                            double* __restrict__ y, double* __restrict__ x) {
+  constexpr int R = kDfBlock * 64 / kDfThreads;  // rows of a wave
+  __shared__ double rb[kDfBlock], zb[kDfBlock], res[kDfBlock], part[4][kDfBlock];
+  const int tid = (int)threadIdx.x, lane = tid & 63;
+  const int nb = n - b0 < kDfBlock ? n - b0 : kDfBlock, i0 = (int)blockIdx.x * kDfBlock + (tid >> 6) * R;
+  double u[R][2];
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+      const int k = lane + 64 * w;
+      u[r][w] = i0 + r < b0 && k < nb ? L[(size_t)(i0 + r) * n + b0 + k] : 0.0;
+    }
+  df_block<false>(L, dinv, n, b0, nb, y, rb, zb, res, part);
+  if (blockIdx.x == 0 && tid < nb) x[b0 + tid] = zb[tid];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    double s = fma(u[r][0], zb[lane], u[r][1] * zb[lane + 64]);
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    if (lane == 0 && i0 + r < b0) y[i0 + r] -= s;
+  }
+}
+
 void launch_df_pack(const double* D, double* d, int n, hipStream_t s) {
   const long long m = (long long)n * (n + 1) / 2;
   if (m > 0) hipLaunchKernelGGL(k_df_pack, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, s, D, d, n);
+}
+
+void launch_df_dots(const double* B, const double* d, size_t np, int naux, double* part, double* x, hipStream_t s) {
+  const int nchunk = (int)df_chunks(np);
+  if (nchunk <= 0 || naux <= 0) return;
+  hipLaunchKernelGGL(k_df_dots, dim3((unsigned)nchunk, (unsigned)((naux + kDfRows - 1) / kDfRows)), dim3(256), 0, s, B,
+                     d, np, naux, nchunk, part);
+  hipLaunchKernelGGL(k_df_sum, dim3((unsigned)((naux + 3) / 4)), dim3(256), 0, s, part, naux, nchunk, x);
+}
+
+void launch_df_inverses(const double* L, int n, double* dinv, hipStream_t s) {
+  if (n > 0)
+    hipLaunchKernelGGL(k_df_inverses, dim3((unsigned)((n + kDfBlock - 1) / kDfBlock)), dim3(kDfBlock), 0, s, L, n, dinv);
+}
+
+void launch_df_solve(const double* L, const double* dinv, int n, double* x, double* y, hipStream_t s) {
+  if (n <= 0) return;
+  for (int b0 = 0; b0 < n; b0 += kDfBlock) {
+    const int below = n - b0 - kDfBlock;
+    hipLaunchKernelGGL(k_df_forward, dim3((unsigned)(below > 0 ? (below + kDfBlock - 1) / kDfBlock : 1)),
+                       dim3(kDfThreads), 0, s, L, dinv, n, b0, x, y);
+  }
+  for (int b0 = (n - 1) / kDfBlock * kDfBlock; b0 >= 0; b0 -= kDfBlock)
+    hipLaunchKernelGGL(k_df_backward, dim3((unsigned)(b0 > 0 ? b0 / kDfBlock : 1)), dim3(kDfThreads), 0, s, L, dinv, n,
+                       b0, y, x);
 }
 
 void launch_df_unpack(const double* j, double* J, int n, hipStream_t s) {

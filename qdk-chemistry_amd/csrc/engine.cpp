@@ -1402,7 +1402,7 @@ static void one_body_device(int device_id);
 // density packed as D_mu,nu + D_nu,mu below the diagonal and D_mu,mu on it.
 struct DFJ {
   int device = 0, nbf = 0, naux = 0;
-  DevBuf<double> B, V, d, x, j, full;
+  DevBuf<double> B, V, d, x, y, j, full, part, dinv;
   rocblas_handle blas = nullptr;
 
   static DFBasisView view(const BasisHost& b, std::vector<DevBuf<int>>& ib, std::vector<DevBuf<double>>& db,
@@ -1440,13 +1440,12 @@ struct DFJ {
     HIP_CHECK(hipMemcpy(full.p, P, sizeof(double) * n * n, hipMemcpyHostToDevice));
     launch_df_pack(full.p, d.p, nbf, nullptr);
     HIP_CHECK(hipGetLastError());
-    const double one = 1.0, zero = 0.0;
+    launch_df_dots(B.p, d.p, np, naux, part.p, x.p, nullptr);
+    HIP_CHECK(hipGetLastError());
+    launch_df_solve(V.p, dinv.p, naux, x.p, y.p, nullptr);
+    HIP_CHECK(hipGetLastError());
     // B is row-major [naux][np], i.e. column-major np x naux
-    if (rocblas_dgemv(blas, rocblas_operation_transpose, (rocblas_int)np, naux, &one, B.p, (rocblas_int)np, d.p, 1,
-                      &zero, x.p, 1) != rocblas_status_success)
-      throw DeviceError("DF-J: rocblas_dgemv failed");
-    if (rocsolver_dpotrs(blas, rocblas_fill_lower, naux, 1, V.p, naux, x.p, naux) != rocblas_status_success)
-      throw DeviceError("DF-J: rocsolver_dpotrs failed");
+    const double one = 1.0, zero = 0.0;
     if (rocblas_dgemv(blas, rocblas_operation_none, (rocblas_int)np, naux, &one, B.p, (rocblas_int)np, x.p, 1, &zero,
                       j.p, 1) != rocblas_status_success)
       throw DeviceError("DF-J: rocblas_dgemv failed");
@@ -1735,6 +1734,9 @@ DFJ::DFJ(const BasisHost& orb, const BasisHost& aux, int dev) : device(dev), nbf
   V.alloc((size_t)naux * naux);
   d.alloc(np);
   j.alloc(np);
+  y.alloc(naux);
+  part.alloc((size_t)naux * df_chunks(np));
+  dinv.alloc((size_t)naux * kDfBlock);
   full.alloc((size_t)nbf * nbf);
   x.alloc(naux);
   launch_df_three_centre(ov, xv, tb.ra, tb.sph, B.p, nullptr);
@@ -1751,6 +1753,9 @@ DFJ::DFJ(const BasisHost& orb, const BasisHost& aux, int dev) : device(dev), nbf
   rocblas_int hinfo = 0;
   HIP_CHECK(hipMemcpy(&hinfo, info.p, sizeof(hinfo), hipMemcpyDeviceToHost));
   if (hinfo != 0) throw std::runtime_error("DF-J: the auxiliary metric is not positive definite");
+  launch_df_inverses(V.p, naux, dinv.p, nullptr);
+  HIP_CHECK(hipGetLastError());
+  HIP_CHECK(hipDeviceSynchronize());
 }
 
 // ------------------------------------------------------------ MO transforms
