@@ -248,9 +248,12 @@ __global__ __launch_bounds__(256) void k_class_stats(const int* __restrict__ cou
 }
 
 __global__ void k_gather_offsets(const long long* __restrict__ offsets, const long long* __restrict__ idx,
-                                 int n, long long* __restrict__ out) {
+                                 int n, const long long* __restrict__ slots, const long long* __restrict__ words,
+                                 long long* __restrict__ out) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) out[i] = offsets[idx[i]];
+  if (i == n) out[n] = slots ? *slots : 0;
+  if (i == n + 1) out[n + 1] = words ? *words : 0;
 }
 
 // ------------------------------------------------------------ symmetrisation
@@ -364,9 +367,9 @@ void launch_sum(void* temp, size_t temp_bytes, const int* in, long long* out, lo
   (void)hipcub::DeviceReduce::Sum(temp, temp_bytes, WideInts(in, WidenInt()), out, (int)n, s);
 }
 
-void launch_gather_offsets(const long long* offsets, const long long* idx, int n, long long* out,
-                           hipStream_t s) {
-  hipLaunchKernelGGL(k_gather_offsets, dim3((n + 63) / 64), dim3(64), 0, s, offsets, idx, n, out);
+void launch_gather_offsets(const long long* offsets, const long long* idx, int n, const long long* slots,
+                           const long long* words, long long* out, hipStream_t s) {
+  hipLaunchKernelGGL(k_gather_offsets, dim3((n + 2 + 63) / 64), dim3(64), 0, s, offsets, idx, n, slots, words, out);
 }
 
 void launch_class_stats(const int* counts, const int2* items, long long nitems, const int* item_cp,

@@ -52,8 +52,9 @@ void launch_exclusive_scan(void* temp, size_t temp_bytes, const int* in, long lo
                            long long n, hipStream_t s);
 // 64-bit sum of n ints (the check of a scan's total); same workspace
 void launch_sum(void* temp, size_t temp_bytes, const int* in, long long* out, long long n, hipStream_t s);
-void launch_gather_offsets(const long long* offsets, const long long* idx, int n, long long* out,
-                           hipStream_t s);
+// out[i] = offsets[idx[i]] for n entries, then *slots and *words (null: zeros)
+void launch_gather_offsets(const long long* offsets, const long long* idx, int n, const long long* slots,
+                           const long long* words, long long* out, hipStream_t s);
 void launch_class_stats(const int* counts, const int2* items, long long nitems, const int* item_cp,
                         const int2* buckets, const PairHdr* pairs, int ncp, double* q_out, double* p_out,
                         hipStream_t s);
