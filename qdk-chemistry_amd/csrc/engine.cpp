@@ -942,18 +942,9 @@ struct Engine {
                       std::abs(lds_max)};
     launch_task_count(sa, counts_d.p, nslot_d.p, nmask_d.p, s);
     HIP_CHECK(hipGetLastError());
-    launch_exclusive_scan(scan_tmp_d.p, scan_tmp_bytes, counts_d.p, offsets_d.p, 2 * nitems + 1, s);
+    launch_task_scans(scan_tmp_d.p, scan_tmp_bytes, counts_d.p, offsets_d.p, slots ? nslot_d.p : nullptr, jslot_d.p,
+                      nmask_d.p, mbase_d.p, sums_d, nitems, s);
     HIP_CHECK(hipGetLastError());
-    launch_sum(scan_tmp_d.p, scan_tmp_bytes, counts_d.p, sums_d, 2 * nitems, s);
-    HIP_CHECK(hipGetLastError());
-    if (slots) {
-      launch_exclusive_scan(scan_tmp_d.p, scan_tmp_bytes, nslot_d.p, jslot_d.p, nitems + 1, s);
-      HIP_CHECK(hipGetLastError());
-      launch_exclusive_scan(scan_tmp_d.p, scan_tmp_bytes, nmask_d.p, mbase_d.p, nitems + 1, s);
-      HIP_CHECK(hipGetLastError());
-      launch_sum(scan_tmp_d.p, scan_tmp_bytes, nslot_d.p, sums_d + 1, nitems, s);
-      HIP_CHECK(hipGetLastError());
-    }
     launch_class_stats(counts_d.p, items_d.p, nitems, item_cp_d.p, buckets_d.p, pairs_d.p, ncp, cstat_d,
                        cstat_d + ncp, s);
     if (mthr >= 0.0)
@@ -1212,18 +1203,15 @@ struct Engine {
     if (det) {
       if (wantJ) Jx_d.alloc(2 * nn);
       if (wantK) Kx_d.alloc(2 * nn);
-      HIP_CHECK(hipMemsetAsync(fxo_d.p, 0, sizeof(int), s));
     }
     for (int idm = 0; idm < ndm; ++idm) {
       double* Jw = wantJ ? dJ[idm] : nullptr;
       double* Kw = wantK ? dK[idm] : nullptr;
-      if (det) {
-        if (Jw) HIP_CHECK(hipMemsetAsync(Jx_d.p, 0, 2 * nn * sizeof(unsigned long long), s));
-        if (Kw) HIP_CHECK(hipMemsetAsync(Kx_d.p, 0, 2 * nn * sizeof(unsigned long long), s));
-      } else {
-        if (Jw) HIP_CHECK(hipMemsetAsync(Jw, 0, nn * sizeof(double), s));
-        if (Kw) HIP_CHECK(hipMemsetAsync(Kw, 0, nn * sizeof(double), s));
-      }
+      if (det)  // 16 bytes an element
+        launch_clear(Jw ? Jx_d.p : nullptr, Kw ? Kx_d.p : nullptr, 2 * nn, idm == 0 ? fxo_d.p : nullptr, s);
+      else
+        launch_clear(Jw, Kw, nn, nullptr, s);
+      HIP_CHECK(hipGetLastError());
       digest(bval, dP[idm], Jw, Kw, kscale, s, nq, nq32);
       if (det) launch_fixed_finish(Jx_d.p, Kx_d.p, Jw, Kw, nbf, 0.25 * kscale, s);
     }

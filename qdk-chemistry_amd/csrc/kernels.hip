@@ -21,9 +21,10 @@ namespace qfe {
 // screens with (compute_shellblock_norm, libint2_direct.cpp:43-59)
 __global__ void k_shell_norm(const double* __restrict__ P, int nbf, const int* __restrict__ sh_bf0,
                              const int* __restrict__ sh_nf, int nsh, double* __restrict__ Pn,
-                             int* __restrict__ bad) {
+                             int* __restrict__ bad, double* __restrict__ pmax) {
   const int s2 = blockIdx.x * blockDim.x + threadIdx.x;
   const int s1 = blockIdx.y;
+  if (s1 == 0 && s2 == 0) *pmax = 0.0;  // k_max_reduce, the next launch, takes the maximum there
   if (s2 >= nsh) return;
   const int r0 = sh_bf0[s1], c0 = sh_bf0[s2], nr = sh_nf[s1], nc = sh_nf[s2];
   double m = 0.0;
@@ -301,8 +302,7 @@ __global__ void k_fixed_finish(const unsigned long long* __restrict__ Jx, const 
 void launch_shell_norm(const double* P, int nbf, const int* sh_bf0, const int* sh_nf, int nsh, double* Pn, int* bad,
                        double* pmax, hipStream_t s) {
   dim3 block(64), grid((nsh + 63) / 64, nsh);
-  hipLaunchKernelGGL(k_shell_norm, grid, block, 0, s, P, nbf, sh_bf0, sh_nf, nsh, Pn, bad);
-  (void)hipMemsetAsync(pmax, 0, sizeof(double), s);
+  hipLaunchKernelGGL(k_shell_norm, grid, block, 0, s, P, nbf, sh_bf0, sh_nf, nsh, Pn, bad, pmax);
   size_t n = (size_t)nsh * nsh;
   int g = (int)((n + 255) / 256);
   if (g > 1024) g = 1024;
@@ -358,13 +358,106 @@ size_t scan_temp_bytes(long long n) {
   return a > b ? a : b;
 }
 
-void launch_exclusive_scan(void* temp, size_t temp_bytes, const int* in, long long* out, long long n,
-                           hipStream_t s) {
+static void launch_exclusive_scan(void* temp, size_t temp_bytes, const int* in, long long* out, long long n,
+                                  hipStream_t s) {
   (void)hipcub::DeviceScan::ExclusiveSum(temp, temp_bytes, WideInts(in, WidenInt()), out, (int)n, s);
 }
 
-void launch_sum(void* temp, size_t temp_bytes, const int* in, long long* out, long long n, hipStream_t s) {
+static void launch_sum(void* temp, size_t temp_bytes, const int* in, long long* out, long long n, hipStream_t s) {
   (void)hipcub::DeviceReduce::Sum(temp, temp_bytes, WideInts(in, WidenInt()), out, (int)n, s);
+}
+
+// One block per array scans it, 4096 elements a step, and its sum is formed
+// apart from the scan.  A small system's screen is a chain of launches (six of
+// them hipcub's, with two kernels each from a few thousand items on): up to
+// kSmallScan elements one launch takes their place (with k_clear for three
+// fills: one water molecule in cc-pVDZ 477 -> 443 us a build).  Beyond, one
+// block's steps of about 1.5 us cost more than the launches.
+struct SmallScan {
+  const int* in;
+  long long* out;
+  long long* sum;  // null: not wanted
+  int n, nsum;     // scanned elements; summed ones
+};
+
+__global__ __launch_bounds__(1024) void k_small_scan(SmallScan a0, SmallScan a1, SmallScan a2) {
+  __shared__ long long wsum[16], ssum[16];
+  const SmallScan a = blockIdx.x == 0 ? a0 : blockIdx.x == 1 ? a1 : a2;
+  const int tid = (int)threadIdx.x, lane = tid & 63, w = tid >> 6;
+  long long carry = 0, own = 0;
+  for (int base = 0; base < a.n; base += 4096) {
+    long long v[4], t = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int i = base + 4 * tid + k;
+      v[k] = i < a.n ? a.in[i] : 0;
+      t += v[k];
+      own += i < a.nsum ? v[k] : 0;
+    }
+    long long inc = t;
+    for (int o = 1; o < 64; o <<= 1) {
+      const long long u = __shfl_up(inc, o);
+      if (lane >= o) inc += u;
+    }
+    if (lane == 63) wsum[w] = inc;
+    __syncthreads();
+    long long ex = carry + inc - t;
+    for (int k = 0; k < 16; ++k) {
+      if (k < w) ex += wsum[k];
+      carry += wsum[k];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int i = base + 4 * tid + k;
+      if (i < a.n) a.out[i] = ex;
+      ex += v[k];
+    }
+    __syncthreads();  // wsum is written again
+  }
+  for (int o = 32; o > 0; o >>= 1) own += __shfl_xor(own, o);
+  if (lane == 0) ssum[w] = own;
+  __syncthreads();
+  if (tid == 0 && a.sum) {
+    long long s = 0;
+    for (int k = 0; k < 16; ++k) s += ssum[k];
+    *a.sum = s;
+  }
+}
+
+void launch_task_scans(void* temp, size_t temp_bytes, const int* counts, long long* offsets, const int* nslot,
+                       long long* jslot, const int* nmask, long long* mbase, long long* sums, long long nitems,
+                       hipStream_t s) {
+  const long long n = 2 * nitems + 1;
+  if (n <= kSmallScan) {
+    const SmallScan a{counts, offsets, sums, (int)n, (int)n - 1};
+    const SmallScan b{nslot, jslot, sums + 1, (int)nitems + 1, (int)nitems};
+    const SmallScan c{nmask, mbase, nullptr, (int)nitems + 1, (int)nitems};
+    hipLaunchKernelGGL(k_small_scan, dim3(nslot ? 3 : 1), dim3(1024), 0, s, a, b, c);
+    return;
+  }
+  launch_exclusive_scan(temp, temp_bytes, counts, offsets, n, s);
+  launch_sum(temp, temp_bytes, counts, sums, n - 1, s);
+  if (!nslot) return;
+  launch_exclusive_scan(temp, temp_bytes, nslot, jslot, nitems + 1, s);
+  launch_exclusive_scan(temp, temp_bytes, nmask, mbase, nitems + 1, s);
+  launch_sum(temp, temp_bytes, nslot, sums + 1, nitems, s);
+}
+
+// the accumulators of a build cleared in one launch
+__global__ __launch_bounds__(256) void k_clear(unsigned long long* __restrict__ a, unsigned long long* __restrict__ b,
+                                               size_t n, int* __restrict__ flag) {
+  const size_t i0 = (size_t)blockIdx.x * 256 + threadIdx.x, step = (size_t)gridDim.x * 256;
+  if (flag && i0 == 0) *flag = 0;
+  if (a)
+    for (size_t i = i0; i < n; i += step) a[i] = 0;
+  if (b)
+    for (size_t i = i0; i < n; i += step) b[i] = 0;
+}
+
+void launch_clear(void* a, void* b, size_t n, int* flag, hipStream_t s) {
+  const size_t g = (n + 255) / 256;
+  hipLaunchKernelGGL(k_clear, dim3((unsigned)(g < 1 ? 1 : g > 4096 ? 4096 : g)), dim3(256), 0, s,
+                     (unsigned long long*)a, (unsigned long long*)b, n, flag);
 }
 
 void launch_gather_offsets(const long long* offsets, const long long* idx, int n, const long long* slots,

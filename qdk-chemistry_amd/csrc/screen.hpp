@@ -45,13 +45,18 @@ void launch_task_count(const ScanArgs& a, int* counts, int* nslot, int* nmask, h
 // its word base mbase[item]
 void launch_task_write(const ScanArgs& a, const int* counts, const long long* offsets, int2* tasks,
                        const long long* mbase, unsigned long long* jmask, hipStream_t s);
-// workspace of launch_exclusive_scan and launch_sum for up to n ints (both
-// accumulate in 64 bits)
+// workspace of launch_task_scans for up to n ints
 size_t scan_temp_bytes(long long n);
-void launch_exclusive_scan(void* temp, size_t temp_bytes, const int* in, long long* out,
-                           long long n, hipStream_t s);
-// 64-bit sum of n ints (the check of a scan's total); same workspace
-void launch_sum(void* temp, size_t temp_bytes, const int* in, long long* out, long long n, hipStream_t s);
+// elements up to which launch_task_scans scans in one launch of its own
+constexpr long long kSmallScan = 32768;
+// exclusive 64-bit scans of counts (2 nitems + 1) and, unless nslot is null,
+// of nslot and nmask (nitems + 1 each), and into sums[0], sums[1] the sums of
+// counts and nslot formed apart from the scans (the check of their totals)
+void launch_task_scans(void* temp, size_t temp_bytes, const int* counts, long long* offsets, const int* nslot,
+                       long long* jslot, const int* nmask, long long* mbase, long long* sums, long long nitems,
+                       hipStream_t s);
+// a and b (null: skipped), n 64-bit words each, and *flag (null: left) to zero
+void launch_clear(void* a, void* b, size_t n, int* flag, hipStream_t s);
 // out[i] = offsets[idx[i]] for n entries, then *slots and *words (null: zeros)
 void launch_gather_offsets(const long long* offsets, const long long* idx, int n, const long long* slots,
                            const long long* words, long long* out, hipStream_t s);
