@@ -9,7 +9,10 @@ operation: FMA = 2, add / mul / hardware rcp / rsq = 1.  The chunk geometry
 of a class evaluates -- is read from the compiled library (qfe_class_chunks,
 i.e. JKChunks of eri_class.hpp itself, including its LDS-row rule), so the
 model follows the kernels that run.  Every chunk kernel repeats the primitive
-loop, so f_prim sums over the chunks.
+loop, so f_prim sums over the chunks.  The model is that of the segment
+kernels (k_eri_jk_seg), which run every class of a large system up to d
+shells; the cooperative kernels (k_eri_jk_coop: few quartets, heavy f classes)
+evaluate each integral once and do less than it counts.
 
 f_prim, per primitive quartet of one chunk:
   setup     PA, PQ (6), p + q (1), rsqrt with two Newton steps (10), rpq (1),
