@@ -72,6 +72,10 @@ __global__ void k_max_reduce(const double* __restrict__ x, size_t n, double* __r
 // quartet it drops fails the exact density test whatever the rounding
 __device__ __forceinline__ double prefix_cut(double thr, double pmax) { return thr / pmax * (1.0 - 1.0e-12); }
 
+// the larger of two numbers that are no NaN (fmax spends an instruction on
+// each operand to make sure)
+__device__ __forceinline__ double nonneg_max(double a, double b) { return a > b ? a : b; }
+
 // One wave scans one item.  pn(c, d) returns max(Pn[a][c], Pn[a][d],
 // Pn[b][c], Pn[b][d]) for the bra shells (a, b); Pcd[q] = Pn of ket pair q.
 //
@@ -107,24 +111,39 @@ __device__ __forceinline__ void scan_item(long long item, int lane, const int2* 
   unsigned long long* const mw = masks ? jmask + mbase[item] : nullptr;
   int c64 = 0, c32 = 0, npre = 0;
   const unsigned long long below = (1ull << lane) - 1ull;
+  // the next step's data is read while this one is tested
+  double Qn = 0.0, pn_q = 0.0;
+  int2 cdn = make_int2(0, 0);
+  auto fetch = [&](int q) {
+    Qn = q < end ? Q[q] : 0.0;
+    if (q < end) {
+      cdn = psh[q];
+      pn_q = Pcd[q];
+    }
+  };
+  fetch(bk.x + lane);
   for (int q0 = bk.x; q0 < end; q0 += 64) {
     const int q = q0 + lane;
-    const double Qq = q < end ? Q[q] : 0.0;
-    // sorted by Q descending: if the first ket (lane 0, q0 < end) fails the
-    // Schwarz bound, all later do
-    if (Qp * __shfl(Qq, 0) < cut) break;
-    bool ok = false, lo = false, pre = false;
-    if (q < end) {
-      pre = !(Qp * Qq < cut);
-      if (pre) {
-        const int2 cd = psh[q];
-        const double m = fmax(fmax(pab, Pcd[q]), pn(cd.x, cd.y));
+    const double Qq = Qn, pcd = pn_q;
+    const int2 cd = cdn;
+    fetch(q + 64);
+    const double qq = Qp * Qq;
+    const bool pre = q < end && !(qq < cut);
+    const unsigned long long mpre = __ballot(pre);
+    if (mpre == 0) break;  // sorted by Q descending: all later kets fail the Schwarz bound too
+    bool ok = false;
+    const bool lo = qq < mix_thr;
+    if (pre) {
+      const double m = nonneg_max(nonneg_max(pab, pcd), pn(cd.x, cd.y));
+      const double t = m * Qp * Qq;
+      ok = !(t < thr);  // libint2_direct.cpp:400-402
+      // within rounding of the threshold the order of the product decides
+      if (fabs(t - thr) <= 1.0e-14 * thr) {
         const int qc1 = cd.x > cd.y ? cd.x : cd.y, qc2 = cd.x > cd.y ? cd.y : cd.x;
         const bool bra_first = pa1 > qc1 || (pa1 == qc1 && pa2 >= qc2);
         const double Q12 = bra_first ? Qp : Qq, Q34 = bra_first ? Qq : Qp;
-        ok = !(m * Q12 * Q34 < thr);  // libint2_direct.cpp:400-402
+        ok = !(m * Q12 * Q34 < thr);
       }
-      lo = Qp * Qq < mix_thr;
     }
     const unsigned long long m64 = __ballot(ok && !lo);
     const unsigned long long m32 = __ballot(ok && lo);
@@ -137,7 +156,7 @@ __device__ __forceinline__ void scan_item(long long item, int lane, const int2* 
     if (masks && lane == 0) mw[(q0 - bk.x) >> 6] = m64 | m32;
     c64 += __popcll(m64);
     c32 += __popcll(m32);
-    npre += __popcll(__ballot(pre));
+    npre += __popcll(mpre);
   }
   if (!WRITE && lane == 0) {
     counts[item] = c64;
@@ -148,9 +167,14 @@ __device__ __forceinline__ void scan_item(long long item, int lane, const int2* 
 }
 
 // One block per segment (the items of one bra pair (a, b) in one class
-// pair): the density-norm rows of a and b are staged in LDS, so the four
-// bra-ket norms of a candidate are LDS reads and only Pcd[q] comes from HBM
-// (coalesced, like Q and psh).  Waves take the segment's items in turn.
+// pair): the larger of the density-norm rows of a and b is staged in LDS, so
+// the four bra-ket norms of a candidate are two LDS reads and only Pcd[q]
+// comes from HBM (coalesced, like Q and psh).  Waves take the segment's items
+// in turn.  The scan is bound by those random LDS reads and by the latency of
+// a step of 64 candidates: with both rows in LDS (four reads) the count took
+// 6.6 and the write 8.8 ms at (H2O)64/cc-pVDZ, with one row and the next step's
+// data read ahead 4.9 and 7.2, and without the product's operand order in the
+// common case 4.6 and 7.0 ms.
 template <bool WRITE>
 __global__ __launch_bounds__(256) void k_task_scan_seg(const int2* __restrict__ segs, const int2* __restrict__ items,
                                                        long long nitems, const int2* __restrict__ buckets,
@@ -164,19 +188,17 @@ __global__ __launch_bounds__(256) void k_task_scan_seg(const int2* __restrict__ 
                                                        const int* __restrict__ cp_nk, int* __restrict__ nslot,
                                                        int* __restrict__ nmask, const long long* __restrict__ mbase,
                                                        unsigned long long* __restrict__ jmask) {
-  extern __shared__ double prow[];  // [2][nsh]: rows a and b of Pn
+  extern __shared__ double prow[];  // [nsh]: max of rows a and b of Pn
   const int2 sg = segs[blockIdx.x];
   const int2 ab = psh[items[sg.x].x];
-  for (int c = threadIdx.x; c < nsh; c += blockDim.x) {
-    prow[c] = Pn[(size_t)ab.x * nsh + c];
-    prow[nsh + c] = Pn[(size_t)ab.y * nsh + c];
-  }
+  for (int c = threadIdx.x; c < nsh; c += blockDim.x)
+    prow[c] = fmax(Pn[(size_t)ab.x * nsh + c], Pn[(size_t)ab.y * nsh + c]);
+  const double pab = Pn[(size_t)ab.x * nsh + ab.y];
   __syncthreads();
-  const double pab = prow[ab.y];
   const double cut = prefix_cut(thr, *pmax_ptr);
   const int nk = cp_nk[item_cp[sg.x]];
   const int lane = (int)(threadIdx.x & 63);
-  auto pn = [&](int c, int d) { return fmax(fmax(prow[c], prow[d]), fmax(prow[nsh + c], prow[nsh + d])); };
+  auto pn = [&](int c, int d) { return nonneg_max(prow[c], prow[d]); };
   for (int item = sg.x + (int)(threadIdx.x >> 6); item < sg.y; item += (int)(blockDim.x >> 6))
     scan_item<WRITE>(item, lane, items, nitems, buckets, pair_bucket, psh, Q, Pcd, pab, ab, pn, cut, thr, mix_thr,
                      counts, offsets, tasks, nk, nslot, nmask, mbase, jmask);
@@ -318,7 +340,7 @@ template <bool WRITE>
 static void task_scan(const ScanArgs& a, int* counts, const long long* offsets, int2* tasks, int* nslot,
                       int* nmask, const long long* mbase, unsigned long long* jmask, hipStream_t s) {
   if (a.nitems <= 0) return;
-  const size_t lds = 2 * sizeof(double) * (size_t)a.nsh;
+  const size_t lds = sizeof(double) * (size_t)a.nsh;
   if (a.segs && a.nseg > 0 && lds <= (size_t)a.lds_max) {
     auto kern = k_task_scan_seg<WRITE>;
     if (lds > 65536) (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
