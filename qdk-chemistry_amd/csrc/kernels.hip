@@ -97,7 +97,8 @@ __device__ __forceinline__ void scan_item(long long item, int lane, const int2* 
                                           const long long* __restrict__ mbase,
                                           unsigned long long* __restrict__ jmask) {
   const bool masks = WRITE && jmask != nullptr;
-  if (WRITE && !masks && counts[item] == 0 && counts[nitems + item] == 0) return;
+  const int total = WRITE ? counts[item] + counts[nitems + item] : 0;
+  if (WRITE && !masks && total == 0) return;
   const int2 it = items[item];
   const int p = it.x;
   const int2 bk = buckets[it.y];
@@ -121,8 +122,11 @@ __device__ __forceinline__ void scan_item(long long item, int lane, const int2* 
       pn_q = Pcd[q];
     }
   };
-  fetch(bk.x + lane);
-  for (int q0 = bk.x; q0 < end; q0 += 64) {
+  if (!WRITE || total > 0) fetch(bk.x + lane);
+  int q0 = bk.x;
+  for (; q0 < end; q0 += 64) {
+    // the write pass knows how many survive, and stops after the last
+    if (WRITE && c64 + c32 == total) break;
     const int q = q0 + lane;
     const double Qq = Qn, pcd = pn_q;
     const int2 cd = cdn;
@@ -158,6 +162,10 @@ __device__ __forceinline__ void scan_item(long long item, int lane, const int2* 
     c32 += __popcll(m32);
     npre += __popcll(mpre);
   }
+  if (masks) {  // the rest of the prefix has no survivor
+    const int words = (int)(mbase[item + 1] - mbase[item]);
+    for (int w = ((q0 - bk.x) >> 6) + lane; w < words; w += 64) mw[w] = 0;
+  }
   if (!WRITE && lane == 0) {
     counts[item] = c64;
     counts[nitems + item] = c32;
@@ -174,7 +182,8 @@ __device__ __forceinline__ void scan_item(long long item, int lane, const int2* 
 // a step of 64 candidates: with both rows in LDS (four reads) the count took
 // 6.6 and the write 8.8 ms at (H2O)64/cc-pVDZ, with one row and the next step's
 // data read ahead 4.9 and 7.2, and without the product's operand order in the
-// common case 4.6 and 7.0 ms.
+// common case 4.6 and 7.0; the write pass stops after an item's last survivor
+// (5.8 ms).
 template <bool WRITE>
 __global__ __launch_bounds__(256) void k_task_scan_seg(const int2* __restrict__ segs, const int2* __restrict__ items,
                                                        long long nitems, const int2* __restrict__ buckets,
