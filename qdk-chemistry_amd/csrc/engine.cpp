@@ -1351,11 +1351,13 @@ static const OneBodyTables& one_body_tables(int device) {
 // flat copy of a basis on the current device, for one call
 struct OneBodyDevice {
   DevBuf<int> l, atom, po, bf0, by_l;
-  DevBuf<double> cen, exps, coefs, Z, R;
+  DevBuf<double> cen, exps, coefs, Z, R, norm;
   OneBodyView view{};
   OneBodyDevice(const BasisHost& b, const double* sph) {
     std::vector<int> hl(b.nsh), hat(b.nsh), hpo(b.nsh + 1, 0), hbf(b.nsh);
-    std::vector<double> hc(3 * (size_t)b.nsh), he, hk;
+    std::vector<double> hc(3 * (size_t)b.nsh), he, hk, hn(b.nsh);
+    double zsum = 0.0;
+    for (double z : b.Z) zsum += std::fabs(z);
     for (int s = 0; s < b.nsh; ++s) {
       const ShellHost& sh = b.shells[s];
       if (sh.l > 3) throw Unsupported("one-electron GPU integrals are compiled for shells up to f");
@@ -1366,6 +1368,16 @@ struct OneBodyDevice {
       he.insert(he.end(), sh.a.begin(), sh.a.end());
       hk.insert(hk.end(), sh.c.begin(), sh.c.end());
       hpo[s + 1] = (int)he.size();
+      // <x^l R | x^l R>: (pi/p)^(3/2) (2l - 1)!! / (2p)^l over primitive pairs
+      double n2 = 0.0;
+      for (size_t i = 0; i < sh.a.size(); ++i)
+        for (size_t j = 0; j < sh.a.size(); ++j) {
+          const double p = sh.a[i] + sh.a[j];
+          double v = sh.c[i] * sh.c[j] * M_PI / p * std::sqrt(M_PI / p);
+          for (int k = 1; k <= sh.l; ++k) v *= (2 * k - 1) / (2.0 * p);
+          n2 += v;
+        }
+      hn[s] = n2 > 0.0 ? std::sqrt(n2) : 0.0;
     }
     std::vector<int> hby(b.nsh);
     std::iota(hby.begin(), hby.end(), 0);
@@ -1380,8 +1392,9 @@ struct OneBodyDevice {
     coefs.upload(hk, nullptr);
     Z.upload(b.Z, nullptr);
     R.upload(b.R, nullptr);
-    view = OneBodyView{l.p, atom.p, po.p, bf0.p, cen.p, exps.p, coefs.p, Z.p, R.p, sph, by_l.p, {0, 0, 0, 0, 0},
-                       b.nsh, b.natoms, b.nbf, b.pure ? 1 : 0};
+    norm.upload(hn, nullptr);
+    view = OneBodyView{l.p, atom.p, po.p, bf0.p, cen.p, exps.p, coefs.p, Z.p, R.p, sph, norm.p, zsum, by_l.p,
+                       {0, 0, 0, 0, 0}, b.nsh, b.natoms, b.nbf, b.pure ? 1 : 0};
     for (int x : hl)
       for (int k = x + 1; k < 5; ++k) ++view.nl[k];
   }

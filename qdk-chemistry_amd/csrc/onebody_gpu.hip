@@ -27,10 +27,14 @@ namespace qfe {
 namespace {
 
 constexpr double kPi1 = 3.14159265358979323846;
-// primitive pairs below this are dropped (|c_a c_b| exp(-ab/p |AB|^2)): their
-// S, T, V and derivative blocks are below it times factors of order
-// (pi/p)^(3/2), the nuclear charges and the angular polynomials
-constexpr double kPairThr = 1e-18;
+// A primitive pair is dropped when no element of its S, T, V or derivative
+// block can reach this times the norms of its two shells (ob_bound).  The
+// prefactor |c_a c_b| exp(-ab/p |AB|^2) alone does not tell: for two f shells
+// of exponent 0.05 at 34 bohr it is 1e-18 and S is 1e-9.  A block sums at most
+// 4096 primitive pairs, so what is dropped stays ten digits below the rounding
+// of an element of order one.  At (H2O)64/cc-pVDZ the cut keeps 29-33 % of the
+// primitive pairs (73 % have a prefactor above the FP64 underflow).
+constexpr double kPairThr = 1e-30;
 
 // shells of pair t of class (LA LB): every ordered combination for LA > LB,
 // the lower triangle for LA == LB
@@ -64,9 +68,30 @@ struct ObPrim {
   double p, PA[3], K, a, b;
 };
 
+// What an element of a primitive pair's cartesian block of operator op (0 = S,
+// 1 = T, 2 = V summed over the nuclei), or of its derivative by a centre, is
+// bounded by.  With r the distance from P a polynomial about A or B is at most
+// (D + r)^l, D = max(|PA|, |PB|), and the n-th moment of D + r over
+// exp(-p r^2), n <= 9, at most (D + 1.75 / sqrt(p))^n = m^n (Minkowski; the
+// ninth root of the ninth moment of r is 1.73 / sqrt(p)); 1/|r - C| is largest
+// for C = P, where the moments are smaller.  The kinetic energy multiplies the
+// second polynomial by lb (lb - 1) / (2 r^2), b (2 lb + 3) and 2 b^2 r^2, a
+// derivative the first by 2a r and la / r, the second by 2b r and lb / r.
+template <int LA, int LB, int op, bool GRAD>
+__device__ double ob_bound(double a, double bb, double AB2, double K, double zsum) {
+  constexpr double lb = LB;
+  const double p = a + bb, m = ((a > bb ? a : bb) * sqrt(AB2) + 1.75 * sqrt(p)) / p, m2 = m * m;
+  double v = fabs(K) * (op == 2 ? 2.0 * kPi1 / p * zsum : kPi1 / p * sqrt(kPi1 / p));
+  for (int i = 0; i < LA + LB; ++i) v *= m;
+  if constexpr (op == 1) v *= 0.5 * lb * (lb - 1.0) / m2 + bb * (2.0 * lb + 3.0) + 2.0 * bb * bb * m2;
+  if constexpr (GRAD) v *= 2.0 * p * m + (LA + LB) / m;
+  return v;
+}
+
 // The significant ones of the primitive pairs [i0, i0 + 64) of (s1, s2),
 // packed into list (64 entries of LDS); returns their number.  Called by the
 // whole one-wave block.
+template <int LA, int LB, int op, bool GRAD>
 __device__ int ob_prims(const OneBodyView& b, int s1, int s2, int i0, int np, ObPrim* list) {
   const int lane = (int)threadIdx.x, i = i0 + lane;
   ObPrim q;
@@ -83,7 +108,8 @@ __device__ int ob_prims(const OneBodyView& b, int s1, int s2, int i0, int np, Ob
     q.p = q.a + q.b;
     for (int d = 0; d < 3; ++d) q.PA[d] = -q.b / q.p * (A[d] - B[d]);
     q.K = exp(-q.a * q.b / q.p * AB2) * (b.coefs[ia] * b.coefs[ib]);
-    keep = fabs(q.K) >= kPairThr;
+    // a NaN is kept
+    keep = q.K != 0.0 && !(ob_bound<LA, LB, op, GRAD>(q.a, q.b, AB2, q.K, b.zsum) < kPairThr * b.norm[s1] * b.norm[s2]);
   }
   const unsigned long long m = __ballot(keep);
   __syncthreads();  // the last list has been read
@@ -185,7 +211,7 @@ __global__ __launch_bounds__(64) void k_one_body(OneBodyView b, RysArgs ra, doub
   double acc[NA * NB];
   sfor<NA * NB>([&](auto k) { acc[k] = 0.0; });
   for (int i0 = 0; i0 < np; i0 += 64) {
-    const int n = ob_prims(b, s1, s2, i0, np, list);
+    const int n = ob_prims<LA, LB, op, false>(b, s1, s2, i0, np, list);
     if constexpr (op <= 1) {
       if (lane < n) {
         const ObPrim q = list[lane];
@@ -314,7 +340,7 @@ __global__ __launch_bounds__(64) void k_one_body_grad_st(OneBodyView b, long lon
     bool have = false;
     double ga[3] = {0.0, 0.0, 0.0}, gb[3] = {0.0, 0.0, 0.0};
     for (int i0 = 0; i0 < np; i0 += 64) {
-      const int n = ob_prims(b, s1, s2, i0, np, list);
+      const int n = ob_prims<LA, LB, op, true>(b, s1, s2, i0, np, list);
       if (n == 0) continue;  // the same for the whole wave
       if (!have) ob_weights<LA, LB>(b, W, s1, s2, wa, wb);
       have = true;
@@ -397,7 +423,7 @@ __global__ __launch_bounds__(64) void k_one_body_grad_v(OneBodyView b, RysArgs r
     bool have = false;
     double ga[3] = {0.0, 0.0, 0.0}, gb[3] = {0.0, 0.0, 0.0};
     for (int i0 = 0; i0 < np; i0 += 64) {
-      const int n = ob_prims(b, s1, s2, i0, np, list);
+      const int n = ob_prims<LA, LB, 2, true>(b, s1, s2, i0, np, list);
       if (n == 0) continue;  // the same for the whole wave
       if (!have) ob_weights<LA, LB>(b, W, s1, s2, wa, wb);
       have = true;

@@ -11,7 +11,9 @@ namespace qfe {
 // range [po[s], po[s+1]) into exps/coefs (normalised contraction
 // coefficients), first output function bf0[s]; per atom the nuclear charge
 // seen by the electrons Z and the position R (3 doubles); the solid-harmonic
-// table sph[l][m][c] (5 x 9 x 15 doubles).  Shells up to l = 3; by_l holds the
+// table sph[l][m][c] (5 x 9 x 15 doubles); per shell the norm of x^l times its
+// radial part, and the sum of the charges' magnitudes zsum (the scales of the
+// cut on primitive pairs).  Shells up to l = 3; by_l holds the
 // shell indices by angular momentum, those of l in [nl[l], nl[l + 1]).
 struct OneBodyView {
   const int* l;
@@ -24,6 +26,8 @@ struct OneBodyView {
   const double* Z;
   const double* R;
   const double* sph;
+  const double* norm;
+  double zsum;
   const int* by_l;
   int nl[5];
   int nsh, natoms, nbf, pure;
