@@ -193,15 +193,19 @@ __device__ int ob_nfun(const OneBodyView& b, int l) { return (b.pure && l >= 2) 
 
 }  // namespace
 
-// S, T or V of one shell pair per block (one wave)
+// S, T or V of one shell pair per block (one wave): pair blockIdx.y gridDim.x +
+// blockIdx.x of the class's npair
 template <int LA, int LB, int op>
-__global__ __launch_bounds__(64) void k_one_body(OneBodyView b, RysArgs ra, double* __restrict__ out) {
+__global__ __launch_bounds__(64) void k_one_body(OneBodyView b, RysArgs ra, long long npair,
+                                                 double* __restrict__ out) {
   constexpr int NA = ncart(LA), NB = ncart(LB), L = LA + LB, NR = L / 2 + 1;
   __shared__ ObPrim list[64];
   __shared__ double blk[NA * NB];
   const int lane = (int)threadIdx.x;
+  const long long t = (long long)blockIdx.y * gridDim.x + blockIdx.x;
+  if (t >= npair) return;
   int s1, s2;
-  ob_pair<LA, LB>(b, blockIdx.x, s1, s2);
+  ob_pair<LA, LB>(b, t, s1, s2);
   const int np = (b.po[s1 + 1] - b.po[s1]) * (b.po[s2 + 1] - b.po[s2]);
   double A[3], B[3];
   for (int d = 0; d < 3; ++d) {
@@ -503,6 +507,9 @@ void ob_classes(F&& f) {
 // waves of a gradient launch: enough to fill the GPU several times over, few
 // enough that their final atomics stay a small part
 constexpr long long kObWaves = 4096;
+// blocks of a matrix launch in x; the rest of a class's pairs go to y, as a
+// dimension of 2^32 threads (2^26 pairs: 11586 s shells) is not run whole
+constexpr long long kObGridX = 1ll << 20;
 
 }  // namespace
 
@@ -510,13 +517,14 @@ void launch_one_body(const OneBodyView& b, const RysArgs& ra, int op, double* ou
   ob_classes([&](auto la, auto lb) {
     const long long n = ob_npairs<la, lb>(b);
     if (n <= 0) return;
-    const dim3 grid((unsigned)n), block(64);
+    const long long gx = std::min(n, kObGridX);
+    const dim3 grid((unsigned)gx, (unsigned)((n + gx - 1) / gx)), block(64);
     if (op == 0)
-      hipLaunchKernelGGL((k_one_body<la, lb, 0>), grid, block, 0, s, b, ra, out);
+      hipLaunchKernelGGL((k_one_body<la, lb, 0>), grid, block, 0, s, b, ra, n, out);
     else if (op == 1)
-      hipLaunchKernelGGL((k_one_body<la, lb, 1>), grid, block, 0, s, b, ra, out);
+      hipLaunchKernelGGL((k_one_body<la, lb, 1>), grid, block, 0, s, b, ra, n, out);
     else
-      hipLaunchKernelGGL((k_one_body<la, lb, 2>), grid, block, 0, s, b, ra, out);
+      hipLaunchKernelGGL((k_one_body<la, lb, 2>), grid, block, 0, s, b, ra, n, out);
   });
 }
 
