@@ -290,13 +290,18 @@ __global__ __launch_bounds__(64) void k_one_body(OneBodyView b, RysArgs ra, long
 // Weights of the derivative of block (s1, s2) in cartesians: wa of the
 // derivative by the first centre (2 W[s1][s2]), wb by the second (2 W[s2][s1],
 // transposed); s1 == s2 is one ordered pair and has the first only.  W of
-// whole-wave blocks, one barrier.
+// whole-wave blocks, one barrier.  diff: the two derivatives are each other's
+// negatives and belong to one atom (S and T of shells on one centre), so their
+// weights go into wa as one difference (half of it where the pair is one) and
+// wb is zero: exactly nothing for a symmetric W, however large 2a makes the
+// terms.  Returns whether a weight of this lane is not zero.
 template <int LA, int LB>
-__device__ void ob_weights(const OneBodyView& b, const double* __restrict__ W, int s1, int s2, double* wa,
+__device__ bool ob_weights(const OneBodyView& b, const double* __restrict__ W, int s1, int s2, bool diff, double* wa,
                            double* wb) {
   constexpr int NA = ncart(LA), NB = ncart(LB);
   const int n1 = ob_nfun(b, LA), n2 = ob_nfun(b, LB), f1 = b.bf0[s1], f2 = b.bf0[s2];
   const size_t n = (size_t)b.nbf;
+  bool any = false;
   __syncthreads();  // the last pair's weights have been read
   for (int k = (int)threadIdx.x; k < NA * NB; k += 64) {
     const int c = k / NB, e = k % NB;
@@ -311,10 +316,13 @@ __device__ void ob_weights(const OneBodyView& b, const double* __restrict__ W, i
         vb = fma(g, W[(size_t)(f2 + j) * n + f1 + i], vb);
       }
     }
+    if (diff) va = (s1 == s2 ? 0.5 : 1.0) * (va - vb);
     wa[k] = va;
-    wb[k] = s1 == s2 ? 0.0 : vb;
+    wb[k] = diff || s1 == s2 ? 0.0 : vb;
+    any = any || va != 0.0 || (!diff && vb != 0.0);
   }
   __syncthreads();
+  return any;
 }
 
 // whether two shells sit on one atom, at one place
@@ -326,7 +334,7 @@ __device__ bool ob_same(const OneBodyView& b, int s1, int s2) {
 
 // S and T derivatives, one wave per block over the pairs of its stride; S and
 // T depend on A - B only, so the second centre's derivative is minus the
-// first's, and a pair on one atom contributes nothing
+// first's, and a pair on one centre contributes what W is not symmetric by
 template <int LA, int LB, int op>
 __global__ __launch_bounds__(64) void k_one_body_grad_st(OneBodyView b, long long npair,
                                                          const double* __restrict__ W, double* __restrict__ grad,
@@ -339,14 +347,14 @@ __global__ __launch_bounds__(64) void k_one_body_grad_st(OneBodyView b, long lon
   for (long long t = blockIdx.x; t < npair; t += gridDim.x) {
     int s1, s2;
     ob_pair<LA, LB>(b, t, s1, s2);
-    if (ob_same(b, s1, s2)) continue;
+    const bool one = ob_same(b, s1, s2);
     const int np = (b.po[s1 + 1] - b.po[s1]) * (b.po[s2 + 1] - b.po[s2]);
     bool have = false;
     double ga[3] = {0.0, 0.0, 0.0}, gb[3] = {0.0, 0.0, 0.0};
     for (int i0 = 0; i0 < np; i0 += 64) {
       const int n = ob_prims<LA, LB, op, true>(b, s1, s2, i0, np, list);
       if (n == 0) continue;  // the same for the whole wave
-      if (!have) ob_weights<LA, LB>(b, W, s1, s2, wa, wb);
+      if (!have && !__any(ob_weights<LA, LB>(b, W, s1, s2, one, wa, wb)) && one) break;
       have = true;
       if (lane >= n) continue;
       const ObPrim q = list[lane];
@@ -429,7 +437,7 @@ __global__ __launch_bounds__(64) void k_one_body_grad_v(OneBodyView b, RysArgs r
     for (int i0 = 0; i0 < np; i0 += 64) {
       const int n = ob_prims<LA, LB, 2, true>(b, s1, s2, i0, np, list);
       if (n == 0) continue;  // the same for the whole wave
-      if (!have) ob_weights<LA, LB>(b, W, s1, s2, wa, wb);
+      if (!have) ob_weights<LA, LB>(b, W, s1, s2, false, wa, wb);
       have = true;
       for (int i = sub; mine && i < n; i += npar) {
         const ObPrim& q = list[i];
