@@ -210,7 +210,7 @@ def gen_sources():
             path = os.path.join(GEN, f"gradc_{tag}.hip")
             _write_if_changed(path, "\n".join(body) + "\n")
             files.append(path)
-            few = "" if fcls else f" && a.ntask <= {grad_coop_tasks(ltot)}"
+            few = "" if fcls else f" && a.coop && a.ntask <= {grad_coop_tasks(ltot)}"
             gr_cases.append(f"  if (cb == {b} && ck == {k}{few}) {{ gradc_cls_{tag}(a, s); return; }}")
             if fcls:
                 continue

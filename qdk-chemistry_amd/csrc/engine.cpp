@@ -279,7 +279,7 @@ struct Engine {
   DevBuf<int> fxo_d;                 // fixed-point range overflow flag
   // primitive-quartet screening at the engine precision (QFE_PRIM_SCREEN=0: off)
   bool prim_screen = true;
-  bool coop = true;                  // QFE_COOP=0: the segment kernels for every class that has them
+  bool coop = true;                  // QFE_COOP=0: the segment / chunk kernels for every class that has them
   int kcol_tile = 0;                 // QFE_KCOL_TILE: cap on the exchange-row tile width
   std::vector<int> sh_bf0_h;         // first function of each shell (+ nbf), host
   std::vector<int> cls_pair_begin;  // first pair of each pair class (pairs are class-sorted)
@@ -852,7 +852,8 @@ struct Engine {
     // QFE_PRIM_SCREEN=0 evaluates every primitive quartet
     if (const char* e = std::getenv("QFE_PRIM_SCREEN"))
       if (e[0] == '0') prim_screen = false;
-    // QFE_COOP=0 runs the segment kernels also where a class has few quartets
+    // QFE_COOP=0 runs the segment kernels of a J/K build and the chunk kernels
+    // of a gradient also where a class has few quartets
     if (const char* e = std::getenv("QFE_COOP"))
       if (e[0] == '0') coop = false;
     // QFE_KCOL_TILE=<columns>: exchange-row tiles of at most that many
@@ -1057,7 +1058,7 @@ struct Engine {
       load[k] += job.first;
       hipStream_t cs = k == 0 ? s : side[k - 1];
       GradLaunch a{tasks_p + bval[cp], bval[cp + 1] - bval[cp], pairs_d.p, ppos_d.p, pk_d.p, pa_d.p, &ra, Pj, Pk,
-                   Pk2, nbf, sh_atom_d.p, natoms, kscale, grad_d.p, grad_d.p + 3 * natoms, kGradCopies, sph_d.p};
+                   Pk2, nbf, sh_atom_d.p, natoms, kscale, grad_d.p, grad_d.p + 3 * natoms, kGradCopies, sph_d.p, coop ? 1 : 0};
       launch_grad(cp_bra[cp], cp_ket[cp], basis.pure, a, cs);
       HIP_CHECK(hipGetLastError());
     }

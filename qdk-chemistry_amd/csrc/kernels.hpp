@@ -100,6 +100,7 @@ struct GradLaunch {
   double* gK;
   int ncopy;              // copies of (gJ, gK) that the blocks spread their atomics over (a power of two)
   const double* sph;      // device copy of the solid-harmonic table kSph (cooperative kernels)
+  int coop;               // 1: classes up to d with few quartets run in the cooperative kernel
 };
 
 struct SchwarzLaunch {
