@@ -530,6 +530,7 @@ struct Engine {
         }
       h.nprim = (int)ppos.size() - h.prim0;
       h.pstride = 1;
+      if (h.nprim == 0) h.prim0 = 0;  // the kernels read a pair's first entry whether it has one or not
     }
     prim_pairs = (long long)ppos.size();
     const int npair = (int)hdr.size();
@@ -595,7 +596,7 @@ struct Engine {
       for (int i = bk.x; i < bk.y; ++i) {
         PairHdr h = hdr[ord[i]];
         const int old0 = h.prim0;
-        h.prim0 = (int)first + (i - bk.x);
+        h.prim0 = h.nprim ? (int)first + (i - bk.x) : 0;
         h.pstride = size;
         std::vector<int> po(h.nprim);
         std::iota(po.begin(), po.end(), 0);
