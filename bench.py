@@ -76,7 +76,7 @@ def timed_builds(eng, P, steps, warmup):
         for prec in (0, 1):
             for cls, nq, npq, ms in eng.class_stats(prec):
                 if nq > 0:
-                    acc = per_class.setdefault((prec, cls), [0.0, 0.0, 0.0, 0])
+                    acc = per_class.setdefault((prec, cls), [0.0, 0.0, 0.0, 0, False])
                     acc[0] += nq
                     acc[2] += ms
                     acc[3] += 1
@@ -87,9 +87,10 @@ def timed_builds(eng, P, steps, warmup):
     # the evaluated primitive quartets (the same in every build of one
     # density), counted after the timed region
     for prec in (0, 1):
-        for cls, nq, npq, ms in eng.class_stats(prec, executed=True):
+        for (cls, nq, npq, ms), coop in zip(eng.class_stats(prec, executed=True), eng.class_cooperative(prec)):
             if (prec, cls) in per_class:
                 per_class[(prec, cls)][1] = npq * per_class[(prec, cls)][3]
+                per_class[(prec, cls)][4] = coop
     n = P.shape[0]
     return dict(seconds=dt, quartets=quartets, quartets_fp32=quartets32, per_class=per_class, stats=eng.stats(),
                 J=eng.download(dJ, (n, n)), K=eng.download(dK, (n, n)))
@@ -122,8 +123,8 @@ def summarize(run, steps):
     dom = None
     dom_total = -1.0
     classes = {}
-    for (prec, cls), (nq, npq, ms, n) in run["per_class"].items():
-        fp, fc = class_flops(*cls)
+    for (prec, cls), (nq, npq, ms, n, coop) in run["per_class"].items():
+        fp, fc = class_flops(*cls, coop=coop)
         f = npq * fp + nq * fc
         classes["(%d%d|%d%d) %s" % (*cls, "fp32" if prec else "fp64")] = dict(
             quartets=nq / steps, prim_quartets=npq / steps, ms=ms / steps, flops=f / steps)
@@ -132,6 +133,8 @@ def summarize(run, steps):
             if ms > dom_total:  # the FP64 class kernel group with the most time
                 dom_total = ms
                 dom = (cls, f / n, nq / n, ms / n)
+        elif coop:  # the cooperative kernels evaluate FP32 tasks in FP64
+            f64 += f
         else:
             f32 += f
     eri_ms = sum(v[2] for v in run["per_class"].values()) / steps
@@ -175,13 +178,14 @@ def log_classes(run, steps, top=12):
     exchange updates the digestion adds into the LDS rows of its segment
     (four K blocks per shell quartet: (na + nb) x (nc + nd) LDS atomics; the
     global atomics are the flushes of those rows, once per non-zero entry and
-    segment, the J_ab block sums and the J_cd tile sums)."""
+    segment, the J_ab block sums and the J_cd tile sums; none for classes in
+    the cooperative kernel, which adds to K in global memory)."""
     from qdk_chemistry_amd.flops import class_flops, nsph
     rows = []
-    for (prec, cls), (nq, npq, ms, n) in run["per_class"].items():
-        fp, fc = class_flops(*cls)
+    for (prec, cls), (nq, npq, ms, n, coop) in run["per_class"].items():
+        fp, fc = class_flops(*cls, coop=coop)
         na, nb, nc, nd = (nsph(x) for x in cls)
-        upd = nq * (na + nb) * (nc + nd)
+        upd = 0.0 if coop else nq * (na + nb) * (nc + nd)
         rows.append((ms / steps, prec, cls, nq / steps, npq / steps, (npq * fp + nq * fc) / (ms * 1e-3) / 1e12,
                      upd / steps))
     rows.sort(reverse=True)

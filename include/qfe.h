@@ -228,8 +228,9 @@ int qfe_get_stats(const qfe_handle* h, qfe_stats* out);
  * cls[4i..4i+3] = (la, lb, lc, ld) as evaluated, quartets[i] and
  * prim_quartets[i] the screened shell quartets and their primitive quartets
  * over significant primitive pairs, exec_prim_quartets[i] (may be NULL) the
- * primitive quartets the kernels evaluated after primitive screening
- * (counted on this call by a counting kernel over the last J/K build's task
+ * primitive quartets the kernels evaluated after primitive screening, each
+ * once (a segment kernel in several chunks evaluates them once a chunk;
+ * counted on this call by a counting kernel over the last J/K build's task
  * list, synchronously on the engine's stream; 0 after a gradient call), and
  * ms[i] the kernel time of that class (the last two only with
  * qfe_config.profile, else 0; a profiled engine launches its class kernels
@@ -237,10 +238,17 @@ int qfe_get_stats(const qfe_handle* h, qfe_stats* out);
  * handle or a failed count.  No reference counterpart: instrumentation. */
 int qfe_class_stats(const qfe_handle* h, int precision, int cap, int* cls, double* quartets,
                     double* prim_quartets, double* exec_prim_quartets, double* ms);
-/* Chunk geometry of the J/K kernels of class (la lb | lc ld) as compiled:
+/* Per class pair in the order of qfe_class_stats: out[i] = 1 where the last J/K
+ * build ran the class's tasks of that precision in the cooperative kernel (a
+ * block per quartet, every integral once, FP64 for the FP32 tasks too), else 0
+ * (segment kernels, or no tasks; all 0 after a gradient call).  Returns n, or
+ * -1 for a null handle.  No reference counterpart: instrumentation. */
+int qfe_class_cooperative(const qfe_handle* h, int precision, int cap, int* out);
+/* Chunk geometry of the segment J/K kernels of class (la lb | lc ld) as compiled:
  * returns the number of chunks n and, for i < min(n, cap), out[4i..4i+3] =
  * the chunk's bra functions [Q0, Q1) and ket cartesians [K0, K1); -1 for a
- * class that is not compiled.  No reference counterpart: instrumentation, the
+ * class that is not compiled; one chunk of the whole quartet for a class that
+ * has the cooperative kernel only.  No reference counterpart: instrumentation, the
  * input of the FLOP model behind the benchmark's roofline. */
 int qfe_class_chunks(int la, int lb, int lc, int ld, int cap, int* out);
 int qfe_nbf(const qfe_handle* h);

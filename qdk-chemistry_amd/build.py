@@ -141,7 +141,7 @@ def gen_sources():
     os.makedirs(GEN, exist_ok=True)
     pcs = pair_classes(MAX_L)
     files = []
-    decls, jk_cases, sw_cases, gr_cases, dn_cases = [], [], [], [], []
+    decls, jk_cases, jc_cases, sw_cases, gr_cases, dn_cases = [], [], [], [], [], []
     head = ["// generated by build.py", '#include "../../eri_grad.hpp"', "namespace qfe {"]
     for b, (la, lb) in enumerate(pcs):
         for k, (lc, ld) in enumerate(pcs[: b + 1]):
@@ -195,8 +195,9 @@ def gen_sources():
                 path = os.path.join(GEN, f"dense_{tag}.hip")
                 _write_if_changed(path, "\n".join(dn) + "\n")
                 files.append(path)
-            few = f" && a.coop && a.ntask <= {jk_coop_tasks(la, lb, lc, ld)}" if seg else ""
-            jk_cases.append(f"  if (cb == {b} && ck == {k}{few}) {{ jkc_cls_{tag}(a, s); return; }}")
+            few = f"coop && ntask <= {jk_coop_tasks(la, lb, lc, ld)}" if seg else "true"
+            jc_cases.append(f"  if (cb == {b} && ck == {k}) return {few};")
+            jk_cases.append(f"  if (cb == {b} && ck == {k}{' && few' if seg else ''}) {{ jkc_cls_{tag}(a, s); return; }}")
             if seg:
                 jk_cases.append(f"  if (cb == {b} && ck == {k}) {{ {' '.join(jk_calls)} return; }}")
             if b == k:
@@ -232,8 +233,10 @@ def gen_sources():
     disp = ["// generated by build.py -- class dispatch", '#include "../../kernels.hpp"',
             '#include "../../eri_dense.hpp"', "#include <stdexcept>",
             "namespace qfe {"] + decls + [
+        "bool jk_cooperative(int cb, int ck, long long ntask, bool coop) {"] + jc_cases + ["  return false;", "}",
         "void launch_jk(int cb, int ck, bool pure, const JKLaunch& a, hipStream_t s) {",
-        '  if (!pure) throw std::runtime_error("cartesian bases are not compiled");'] + jk_cases + [
+        '  if (!pure) throw std::runtime_error("cartesian bases are not compiled");',
+        "  const bool few = jk_cooperative(cb, ck, a.ntask, a.coop != 0);"] + jk_cases + [
         '  throw std::runtime_error("ERI class not compiled");', "}",
         "void launch_schwarz(int c, bool pure, const SchwarzLaunch& a, hipStream_t s) {",
         '  if (!pure) throw std::runtime_error("cartesian bases are not compiled");'] + sw_cases + [

@@ -1259,9 +1259,18 @@ struct Engine {
     stats.ms_total = t03;
   }
 
+  // whether the last J/K build ran a class (FP64 or FP32 tasks) in the
+  // cooperative kernel, as launch_jk decided
+  bool ran_coop(int prec, int cp) const {
+    const size_t n = cp_bra.size();
+    if (last_bval.size() != 2 * (n + 1)) return false;
+    const long long* b = last_bval.data() + prec * (n + 1);
+    return b[cp + 1] > b[cp] && jk_cooperative(cp_bra[cp], cp_ket[cp], b[cp + 1] - b[cp], coop);
+  }
+
   // the primitive quartets the class kernels evaluated in the last J/K build
   // (profiled engines; zeros otherwise, or after a gradient replaced the
-  // task list): the same prefix walk, without the integrals, outside any
+  // task list): the kernels' own walks, without the integrals, outside any
   // timed build
   void count_executed() const {
     if (pqc_valid) return;
@@ -1274,7 +1283,7 @@ struct Engine {
         const long long* b = last_bval.data() + prec * (ncp + 1);
         for (int cp = 0; cp < ncp; ++cp)
           launch_count_prims(tasks_p + b[cp], b[cp + 1] - b[cp], pairs_d.p, sig_d.p, sig32_d.p, pmax_d.p,
-                             prim_screen ? 1 : 0, prec, pqc_d.p + (size_t)prec * ncp + cp, stream);
+                             prim_screen ? 1 : 0, prec, ran_coop(prec, cp) ? 1 : 0, pqc_d.p + (size_t)prec * ncp + cp, stream);
       }
       HIP_CHECK(hipGetLastError());
       HIP_CHECK(hipMemcpyAsync(pqc_h.data(), pqc_d.p, sizeof(unsigned long long) * 2 * ncp, hipMemcpyDeviceToHost,
@@ -1667,6 +1676,13 @@ int qfe_class_stats(const qfe_handle* h, int precision, int cap, int* cls, doubl
     if (exec_prim_quartets)
       exec_prim_quartets[cp] = e.pqc_h.empty() ? 0.0 : (double)e.pqc_h[(precision ? ncp : 0) + cp];
   }
+  return ncp;
+}
+
+int qfe_class_cooperative(const qfe_handle* h, int precision, int cap, int* out) {
+  if (!h) return -1;
+  const int ncp = (int)h->e.cp_bra.size();
+  for (int cp = 0; cp < ncp && cp < cap; ++cp) out[cp] = h->e.ran_coop(precision ? 1 : 0, cp) ? 1 : 0;
   return ncp;
 }
 

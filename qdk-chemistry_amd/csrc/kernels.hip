@@ -697,19 +697,19 @@ void launch_copy_words(const unsigned long long* src, unsigned long long* dst, s
 template <typename R>
 __global__ __launch_bounds__(256) void k_count_prims(const int2* __restrict__ tasks, long long ntask,
                                                      const PairHdr* __restrict__ pairs, const R* __restrict__ sig,
-                                                     const double* __restrict__ pmax,
-                                                     int prim_screen, unsigned long long* __restrict__ count) {
+                                                     const double* __restrict__ pmax, int prim_screen, int coop,
+                                                     unsigned long long* __restrict__ count) {
   const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   unsigned long long n = 0;
   if (t < ntask) {
     const int2 tk = tasks[t];
     const PairHdr bra = pairs[tk.x], ket = pairs[tk.y];
     const R lnp = prim_ln_cut<R>(pmax, prim_screen);
-    const R sb0 = sig[bra.prim0];
+    const R sb0 = sig[bra.prim0], sk0 = sig[ket.prim0];
     for (int ik = ket.prim0; ik < ket.prim0 + ket.nprim * ket.pstride; ik += ket.pstride) {
       const R sk = sig[ik];
       if (sk + sb0 < lnp) break;
-      const R blim = lnp - sk;
+      const R blim = lnp - (coop ? sk0 : sk);
       for (int ib = bra.prim0; ib < bra.prim0 + bra.nprim * bra.pstride; ib += bra.pstride) {
         if (sig[ib] < blim) break;
         ++n;
@@ -722,16 +722,16 @@ __global__ __launch_bounds__(256) void k_count_prims(const int2* __restrict__ ta
 }
 
 void launch_count_prims(const int2* tasks, long long ntask, const PairHdr* pairs, const double* sig,
-                        const float* sig32, const double* pmax, int prim_screen, int fp32,
+                        const float* sig32, const double* pmax, int prim_screen, int fp32, int coop,
                         unsigned long long* count, hipStream_t s) {
   if (ntask <= 0) return;
   const dim3 grid((unsigned)((ntask + 255) / 256));
-  if (fp32)
+  if (fp32 && !coop)
     hipLaunchKernelGGL(k_count_prims<float>, grid, dim3(256), 0, s, tasks, ntask, pairs, sig32, pmax,
-                       prim_screen, count);
+                       prim_screen, coop, count);
   else
     hipLaunchKernelGGL(k_count_prims<double>, grid, dim3(256), 0, s, tasks, ntask, pairs, sig, pmax,
-                       prim_screen, count);
+                       prim_screen, coop, count);
 }
 
 }  // namespace qfe

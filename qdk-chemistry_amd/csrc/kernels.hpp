@@ -113,6 +113,9 @@ struct SchwarzLaunch {
   double* q2;
 };
 
+// whether launch_jk runs ntask tasks of a class in the cooperative kernel
+// (coop = false: only a class that has no segment kernels)
+bool jk_cooperative(int bra_cls, int ket_cls, long long ntask, bool coop);
 void launch_jk(int bra_cls, int ket_cls, bool pure, const JKLaunch& a, hipStream_t s);
 void launch_schwarz(int pair_cls, bool pure, const SchwarzLaunch& a, hipStream_t s);
 void launch_grad(int bra_cls, int ket_cls, bool pure, const GradLaunch& a, hipStream_t s);

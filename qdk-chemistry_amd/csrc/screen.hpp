@@ -84,12 +84,13 @@ void launch_fixed_finish(const unsigned long long* Jx, const unsigned long long*
                          double kq, hipStream_t s);
 // g[i] = sum of its ncopy copies, n apart (the gradient's accumulators)
 void launch_fold_copies(double* g, int n, int ncopy, hipStream_t s);
-// Profiling: add to *count the primitive quartets that the class kernels
-// evaluate for the tasks [0, ntask): the same prefix walk over primitives
-// sorted by sig, in the same precision and with the same cut, without the
-// integrals
+// Profiling: add to *count the primitive quartets that the J/K kernels evaluate
+// for the tasks [0, ntask), without the integrals: the prefix walk of the
+// segment kernels over primitives sorted by sig, in the same precision and
+// with the same cut, or (coop) the full product of the two prefixes that the
+// cooperative kernels evaluate, in FP64 whatever fp32 says.
 void launch_count_prims(const int2* tasks, long long ntask, const PairHdr* pairs, const double* sig,
-                        const float* sig32, const double* pmax, int prim_screen, int fp32,
+                        const float* sig32, const double* pmax, int prim_screen, int fp32, int coop,
                         unsigned long long* count, hipStream_t s);
 constexpr int kJcdTileBra = 256;   // bra pairs per tile, at most
 constexpr int kJcdTileKet = 1024;  // ket positions per tile, at most (a multiple of 64)

@@ -43,7 +43,7 @@ EXPORTS = ["qfe_create", "qfe_build_jk", "qfe_build_jk_device", "qfe_gradients",
            "qfe_one_body_grad", "qfe_one_body_gpu", "qfe_one_body_grad_gpu", "qfe_eigh_gpu",
            "qfe_dfj_create", "qfe_dfj_build_j", "qfe_dfj_naux", "qfe_dfj_destroy",
            "qfe_quarter_trans", "qfe_mo_eri", "qfe_scf_create", "qfe_scf_set_density",
-           "qfe_scf_step", "qfe_scf_update", "qfe_scf_finish", "qfe_scf_get", "qfe_scf_destroy", "qfe_get_stats", "qfe_class_stats", "qfe_build_jk_device_noalloc", "qfe_noalloc_scratch_bytes", "qfe_set_precision", "qfe_device_buffers", "qfe_copy", "qfe_class_chunks", "qfe_nbf", "qfe_max_l", "qfe_destroy",
+           "qfe_scf_step", "qfe_scf_update", "qfe_scf_finish", "qfe_scf_get", "qfe_scf_destroy", "qfe_get_stats", "qfe_class_stats", "qfe_class_cooperative", "qfe_build_jk_device_noalloc", "qfe_noalloc_scratch_bytes", "qfe_set_precision", "qfe_device_buffers", "qfe_copy", "qfe_class_chunks", "qfe_nbf", "qfe_max_l", "qfe_destroy",
            "qfe_last_error"]
 
 _lib = None
@@ -100,6 +100,7 @@ def lib():
         L.qfe_device_buffers.argtypes = [ctypes.c_void_p, ctypes.POINTER(ctypes.c_void_p),
                                          ctypes.POINTER(ctypes.c_void_p), ctypes.POINTER(ctypes.c_void_p)]
         L.qfe_copy.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_ulonglong, ctypes.c_int]
+        L.qfe_class_cooperative.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, _ip]
         L.qfe_class_stats.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, _ip, _dp, _dp, _dp, _dp]
         L.qfe_class_chunks.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, _ip]
         L.qfe_nbf.argtypes = [ctypes.c_void_p]

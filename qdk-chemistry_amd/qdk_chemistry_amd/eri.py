@@ -166,6 +166,14 @@ class RysERI:
         return [(tuple(int(x) for x in cls[4 * i:4 * i + 4]), float(q[i]), float(p[i]), float(ms[i]))
                 for i in range(min(n, cap))]
 
+    def class_cooperative(self, precision=0):
+        """Per row of class_stats(precision): whether the last J/K build ran
+        that class in the cooperative kernel."""
+        cap = 256
+        out = np.zeros(cap, dtype=np.int32)
+        n = _lib.lib().qfe_class_cooperative(self.h, precision, cap, _lib.ptr(out, ctypes.c_int))
+        return [bool(x) for x in out[:max(0, min(n, cap))]]
+
     def stats(self) -> dict:
         s = _lib.QfeStats()
         _lib.check(_lib.lib().qfe_get_stats(self.h, ctypes.byref(s)))

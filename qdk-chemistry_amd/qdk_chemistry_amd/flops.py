@@ -9,10 +9,10 @@ operation: FMA = 2, add / mul / hardware rcp / rsq = 1.  The chunk geometry
 of a class evaluates -- is read from the compiled library (qfe_class_chunks,
 i.e. JKChunks of eri_class.hpp itself, including its LDS-row rule), so the
 model follows the kernels that run.  Every chunk kernel repeats the primitive
-loop, so f_prim sums over the chunks.  The model is that of the segment
-kernels (k_eri_jk_seg), which run every class of a large system up to d
-shells; the cooperative kernels (k_eri_jk_coop: few quartets, heavy f classes)
-evaluate each integral once and do less than it counts.
+loop, so f_prim sums over the chunks.  That is the model of the segment
+kernels (k_eri_jk_seg); a class that a build ran in the cooperative kernel
+(k_eri_jk_coop: few quartets, heavy f classes; qfe_class_cooperative) is
+counted with coop=True, every integral once.
 
 f_prim, per primitive quartet of one chunk:
   setup     PA, PQ (6), p + q (1), rsqrt with two Newton steps (10), rpq (1),
@@ -33,6 +33,14 @@ f_contr, per shell quartet and chunk: the ket solid-harmonic transform
 scaling and 6 FMAs per bra function x ket function), plus 20 for the task
 set-up.  The ket-primitive work of the outer loop (amortised over the bra
 primitives) is not counted.
+
+With coop, f_prim is the same set-up, roots, recursions and transfers, once
+(the three lanes of a combination repeat the set-up and the root: not counted),
+and 1 mul and 1 FMA per cartesian component of the quartet and root; f_contr
+the four transforms to solid harmonics (1 FMA per nonzero coefficient and
+element of the other indices; indices below d are copied) and six contractions
+of the block with a density block (1 FMA per element each), the deg scaling of
+their outputs and 20 for the task set-up.
 """
 from __future__ import annotations
 
@@ -131,9 +139,26 @@ def _per_root(EA, FC):
             (1 + 6 if EA else 0) + (1 + 6 if FC else 0) + 1)
 
 
+def _coop_flops(la, lb, lc, ld, pure):
+    """(f_prim, f_contr) of the cooperative kernel."""
+    L = la + lb + lc + ld
+    nr, EA, FC = L // 2 + 1, la + lb, lc + ld
+    ls = (la, lb, lc, ld)
+    na, nb, nc, nd = (ncart(x) for x in ls)
+    ma, mb, mc, md = (nsph(x, pure) for x in ls)
+    f_prim = _setup(EA, FC) + _roots(nr, L) + nr * (_per_root(EA, FC) + 3 * _onedim(la, lb, lc, ld) + 3 * na * nb * nc * nd)
+    nnz = [2 * int(np.count_nonzero(_sph(x, pure))) if nsph(x, pure) != ncart(x) else 0 for x in ls]
+    f_contr = (na * nb * nc * nnz[3] + na * nb * md * nnz[2] + na * mc * md * nnz[1] + mb * mc * md * nnz[0] +
+               12 * ma * mb * mc * md + ma * mb + mc * md + (ma + mb) * (mc + md) + 20)
+    return f_prim, f_contr
+
+
 @lru_cache(maxsize=None)
-def class_flops(la, lb, lc, ld, pure=True):
-    """(f_prim, f_contr) for class (la lb | lc ld) as compiled."""
+def class_flops(la, lb, lc, ld, pure=True, coop=False):
+    """(f_prim, f_contr) for class (la lb | lc ld) as compiled, in its segment
+    kernels or (coop) in its cooperative kernel."""
+    if coop:
+        return _coop_flops(la, lb, lc, ld, pure)
     L = la + lb + lc + ld
     nr = L // 2 + 1
     Sa, Sb, Sc, Sd = _sph(la, pure), _sph(lb, pure), _sph(lc, pure), _sph(ld, pure)
@@ -163,7 +188,8 @@ def class_flops(la, lb, lc, ld, pure=True):
 
 
 def build_flops(class_rows):
-    """class_rows: iterable of ((la, lb, lc, ld), quartets, prim_quartets)."""
+    """class_rows: iterable of ((la, lb, lc, ld), quartets, prim_quartets), all
+    in segment kernels."""
     tot = 0.0
     for cls, nq, npq in class_rows:
         fp, fc = class_flops(*cls)
