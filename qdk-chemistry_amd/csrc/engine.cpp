@@ -1362,11 +1362,11 @@ static const OneBodyTables& one_body_tables(int device) {
 // flat copy of a basis on the current device, for one call
 struct OneBodyDevice {
   DevBuf<int> l, atom, po, bf0, by_l;
-  DevBuf<double> cen, exps, coefs, Z, R, norm;
+  DevBuf<double> cen, exps, coefs, Z, R;  // cen: centres, then the shells' norms
   OneBodyView view{};
   OneBodyDevice(const BasisHost& b, const double* sph) {
     std::vector<int> hl(b.nsh), hat(b.nsh), hpo(b.nsh + 1, 0), hbf(b.nsh);
-    std::vector<double> hc(3 * (size_t)b.nsh), he, hk, hn(b.nsh);
+    std::vector<double> hc(4 * (size_t)b.nsh), he, hk;
     double zsum = 0.0;
     for (double z : b.Z) zsum += std::fabs(z);
     for (int s = 0; s < b.nsh; ++s) {
@@ -1388,7 +1388,7 @@ struct OneBodyDevice {
           for (int k = 1; k <= sh.l; ++k) v *= (2 * k - 1) / (2.0 * p);
           n2 += v;
         }
-      hn[s] = n2 > 0.0 ? std::sqrt(n2) : 0.0;
+      hc[3 * (size_t)b.nsh + s] = n2 > 0.0 ? std::sqrt(n2) : 0.0;
     }
     std::vector<int> hby(b.nsh);
     std::iota(hby.begin(), hby.end(), 0);
@@ -1403,9 +1403,9 @@ struct OneBodyDevice {
     coefs.upload(hk, nullptr);
     Z.upload(b.Z, nullptr);
     R.upload(b.R, nullptr);
-    norm.upload(hn, nullptr);
-    view = OneBodyView{l.p, atom.p, po.p, bf0.p, cen.p, exps.p, coefs.p, Z.p, R.p, sph, norm.p, zsum, by_l.p,
-                       {0, 0, 0, 0, 0}, b.nsh, b.natoms, b.nbf, b.pure ? 1 : 0};
+    view = OneBodyView{l.p, atom.p, po.p, bf0.p, cen.p, exps.p, coefs.p, Z.p, R.p, sph,
+                       cen.p + 3 * (size_t)b.nsh, zsum, by_l.p, {0, 0, 0, 0, 0}, b.nsh, b.natoms, b.nbf,
+                       b.pure ? 1 : 0};
     for (int x : hl)
       for (int k = x + 1; k < 5; ++k) ++view.nl[k];
   }
