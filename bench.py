@@ -328,7 +328,7 @@ def c20h42_scf(mix_threshold=1e-6):
 
 def gradient_timings(systems=("h2o16", "c20h42")):
     """The ERI gradient (adjoint kernels) of the gradient configurations,
-    (H2O)16/cc-pVDZ and C20H42/cc-pVTZ (f shells: the generic kernel), at
+    (H2O)16/cc-pVDZ and C20H42/cc-pVTZ (f shells: cooperative kernels), at
     the atomic-guess density: one warm-up, then one timed call each."""
     from qdk_chemistry_amd.basis import load_basis
     from qdk_chemistry_amd.eri import ERIConfig, create

@@ -63,8 +63,9 @@ typedef struct {
   int mix_precision;           /* 1: FP32 for quartets whose Schwarz bound < mix_threshold */
   double mix_threshold;        /* 1e-6 */
   int verbose;
-  int profile;                 /* 1: time every class kernel group with HIP events (its class kernels then
-                                  run one after another; else they spread over QFE_STREAMS streams) */
+  int profile;                 /* 1: time every class kernel group of a J/K build with HIP events (its class
+                                  kernels then run one after another; else, and in gradients, they spread
+                                  over QFE_STREAMS streams) */
   int use_atomics;             /* 0 (the reference's default, core/scf.h:81-82): bitwise-repeatable
                                   J/K (order-independent fixed-point accumulation); 1: FP64 atomics */
 } qfe_config;

@@ -214,7 +214,7 @@ __global__ __launch_bounds__(256) void k_task_scan_seg(const int2* __restrict__ 
 }
 
 // The same scan with one wave per item and the norms gathered from HBM (for
-// shell counts whose two rows do not fit the LDS).
+// shell counts whose row does not fit the LDS).
 template <bool WRITE>
 __global__ __launch_bounds__(256) void k_task_scan(const int2* __restrict__ items, long long nitems,
                                                    const int2* __restrict__ buckets,

@@ -14,7 +14,8 @@
 // cartesian block (V) or its nucleus's forces (the V gradient) in registers.
 // The kernels are bound by the FP64 work of those combinations; a thread per
 // pair with runtime angular momenta kept its tables in 4-6 KB of scratch a
-// lane: V took 13 ms and its gradient 14.6 ms at (H2O)24/cc-pVDZ.
+// lane: V took 13 ms and its gradient 14.6 ms at (H2O)24/cc-pVDZ, 0.15 and
+// 0.37 ms now.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
